@@ -63,6 +63,10 @@ gr_status_t launch_mfma_prefill(const DecodeArgs& a, hipStream_t stream);
 // Split-prefix decode (a.nsplit > 1, workspace set): the decode kernel, then
 // the merge of its partials.
 gr_status_t launch_mfma_decode_split(const DecodeArgs& a, hipStream_t stream);
+// 512-byte rows (gr_attn_row512.hip): float32 at head_dim 128, bf16/fp16 at
+// head_dim 256, 16-byte aligned, no window, ALiBi or fp8 cache.
+bool row512_decode_supported(const DecodeArgs& a);
+gr_status_t launch_row512_decode(const DecodeArgs& a, hipStream_t stream);
 // Row tiles of the MFMA decode grid and the prefix split it would use.
 void mfma_decode_plan(int num_reqs, int max_beams, int q_per_beam, int Hq, int Hkv, int max_prefix_len,
                       int* tiles, int* nsplit);

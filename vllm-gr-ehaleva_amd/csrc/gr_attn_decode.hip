@@ -5,7 +5,9 @@
 // flash-attention prefix pass, a Triton suffix gather, a suffix pass and an
 // LSE merge (vllm_gr/v1/attention/backends/beam_attn.py:629-701).
 //
-// Two kernels sit behind gr_beam_attn_decode:
+// Three kernels sit behind gr_beam_attn_decode:
+//  * decode_row512 (gr_attn_row512.hip): 512-byte rows (float32 at head_dim
+//    128, bf16/fp16 at head_dim 256) without window, ALiBi or fp8 cache.
 //  * decode_generic: any dtype (fp32/fp16/bf16), head_dim % 8 == 0 <= 256.
 //    One workgroup per (request, KV head, 32-row chunk of the request's beam
 //    rows): the chunk's beams share each prefix tile; fp32 VALU math.
@@ -514,6 +516,7 @@ extern "C" gr_status_t gr_beam_attn_decode(
     if (mfma_decode_supported(a)) return launch_mfma_decode(a, stream);
     DecodeArgs p;
     if (mfma_pair_args(a, p)) return launch_mfma_decode(p, stream);
+    if (row512_decode_supported(a)) return launch_row512_decode(a, stream);
   }
   return launch_generic<false>(a, stream);
 }
@@ -565,6 +568,7 @@ static gr_status_t decode_ws_impl(
   if (g_decode_kernel_override != 1 && !mfma_decode_supported(a)) {
     DecodeArgs p;  // head_dim 64 as head pairs, never split (the workspace is for head_dim 128)
     if (mfma_pair_args(a, p)) return launch_mfma_decode(p, stream);
+    if (row512_decode_supported(a)) return launch_row512_decode(a, stream);
   }
   if (g_decode_kernel_override == 1 || !mfma_decode_supported(a)) return launch_generic<false>(a, stream);
   int tiles, nsplit;

@@ -1,0 +1,475 @@
+// BeamAttention decode on the matrix cores for 512-byte K / V rows (float32 at
+// head_dim 128, bf16 / fp16 at head_dim 256), in float32 precision throughout.
+//
+// What bounds it: these shapes are small (tens of megabytes of KV at most a
+// request), so the time is the chain of one workgroup: its share of the keys
+// through the CU's 64 bytes per clock, or, in float32, the float32 MFMA rate.
+// The split is therefore over rows and, inside the workgroup, over keys: a
+// workgroup owns 16 query rows of one (request, KV head) -- the smallest MFMA
+// tile, for the most workgroups -- and its 8 waves take every eighth tile of 32
+// keys, each with its own online softmax; the eight partial states meet in LDS
+// at the end.  No second launch and no workspace.  Workgroups of one (request,
+// KV head) sit on one XCD and share its L2.
+//
+// Formulation (v_mfma_f32_16x16x32_{bf16,f16}, v_mfma_f32_16x16x4_f32), lane =
+// (quarter g, m = lane % 16):
+//   S^T[key][row] = K . Q^T   A = K rows from LDS, B = Q rows (registers)
+//   O^T[d][row]  += V^T . P^T A = V (registers), B = P as the S^T accumulators hold it
+// The contraction index of an MFMA may be numbered at will as long as both
+// operands agree, which saves every layout change but one:
+//  * QK: step j contracts the 16-byte chunks 4 j + g of a row;
+//  * PV: an accumulator register (block kb, r) of quarter g is key 16 kb + 4 g +
+//    r, so a lane loads V rows of exactly these keys (8 of the tile's 32), 16
+//    bytes at chunk 16 c + m, and output block (c, e) is dim PER (16 c + m) + e.
+//    float32 values are operands as loaded; 16-bit ones need an 8 x 8 transpose
+//    inside the lane (32 byte permutes per chunk).
+// K tiles go straight from global memory into the wave's own LDS tile (chunks
+// XOR-swizzled by the key, so the A reads touch every bank once); the next
+// tile's transfer runs under this tile's softmax and PV, and V arrives in
+// registers under QK.  No barrier inside the loop: a wave reads only its own
+// tiles.
+//
+// Measured (MI355X, whole call, the generic kernel -> this one): float32, 1
+// request x 32 beams, 512-token prompt, 16 / 4 heads: 174.6 -> 21.7 us; bf16
+// head_dim 256, 4 requests x 64 beams, 1024-token prompts, 16 / 8 heads, soft
+// cap: 557 -> 25.1 us.  Error against float64: 5.7e-7 -> 4.2e-7 and 1.7e-3
+// (output rounding) both.
+//
+// Precision: scores, probabilities and sums are float32.  A 16-bit PV takes
+// each probability as two 16-bit terms (hi + lo, 16 bits of it), two MFMAs.
+#include "gr_mfma_tile.h"
+
+namespace gr {
+namespace {
+
+constexpr int R5_THREADS = 512;
+constexpr int R5_WAVES = R5_THREADS / 64;
+constexpr int R5_ROWS = 16;      // query rows per workgroup
+constexpr int R5_KEYS = 32;      // keys per wave tile
+constexpr int R5_BYTES = 512;    // one K / V row
+constexpr int R5_TILE = R5_KEYS * R5_BYTES;
+
+typedef float f4_t __attribute__((__vector_size__(16)));
+
+template <int DT> struct Row512;
+template <> struct Row512<GR_DTYPE_F32> {
+  static constexpr int PER = 4;  // elements per 16-byte chunk
+  static constexpr float PSCALE = 1.f;
+  __device__ static inline f4_t qk(u32x4_t k, u32x4_t q, f4_t s) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(k[e]), __uint_as_float(q[e]), s, 0, 0, 0);
+    return s;
+  }
+  __device__ static inline u32x4_t pack(const float (&v)[4]) {
+    return u32x4_t{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
+  }
+};
+template <> struct Row512<GR_DTYPE_BF16> {
+  static constexpr int PER = 8;
+  static constexpr float PSCALE = 1.f;
+  __device__ static inline f4_t mma(u32x4_t a, u32x4_t b, f4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
+                                                   0, 0, 0);
+  }
+  __device__ static inline f4_t qk(u32x4_t k, u32x4_t q, f4_t s) { return mma(k, q, s); }
+  // p = hi + lo with both terms positive for p > 0, so that an infinite V row
+  // gives the infinity that a float32 weight gives it: hi is cut off (not
+  // rounded) from just below p, lo is at least 2^-9 p
+  __device__ static inline void split(float p, float& hi, float& lo) {
+    hi = __uint_as_float(__float_as_uint(p * 0x1.ffp-1f) & 0xffff0000u);
+    lo = p - hi;
+  }
+  __device__ static inline u32x4_t pack(const float (&v)[8]) {
+    return u32x4_t{Mma<GR_DTYPE_BF16>::pack2(v[0], v[1]), Mma<GR_DTYPE_BF16>::pack2(v[2], v[3]),
+                   Mma<GR_DTYPE_BF16>::pack2(v[4], v[5]), Mma<GR_DTYPE_BF16>::pack2(v[6], v[7])};
+  }
+};
+template <> struct Row512<GR_DTYPE_F16> {
+  static constexpr int PER = 8;
+  // weights are carried as 256 p (at most 256): the low terms stay normal
+  static constexpr float PSCALE = 256.f;
+  __device__ static inline f4_t mma(u32x4_t a, u32x4_t b, f4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0,
+                                                  0, 0);
+  }
+  __device__ static inline f4_t qk(u32x4_t k, u32x4_t q, f4_t s) { return mma(k, q, s); }
+  // as for bf16; a term below fp16's range stays at its smallest value
+  // (2^-32 of the row's largest weight)
+  __device__ static inline void split(float p, float& hi, float& lo) {
+    hi = (float)(_Float16)(p * 0x1.ffp-1f);
+    hi = p > 0.f ? fmaxf(hi, 0x1p-24f) : hi;
+    lo = p > 0.f ? fmaxf(p - hi, 0x1p-24f) : p - hi;
+  }
+  __device__ static inline u32x4_t pack(const float (&v)[8]) {
+    return u32x4_t{Mma<GR_DTYPE_F16>::pack2(v[0], v[1]), Mma<GR_DTYPE_F16>::pack2(v[2], v[3]),
+                   Mma<GR_DTYPE_F16>::pack2(v[4], v[5]), Mma<GR_DTYPE_F16>::pack2(v[6], v[7])};
+  }
+};
+
+// The row's partial outputs of one wave in LDS: 16 rows of PER * 32 floats, 16
+// bytes of padding a row (rows start on different banks).
+template <int PER> constexpr int r5_pitch() { return PER * 32 + 4; }
+template <int PER> constexpr int r5_region() {
+  return R5_ROWS * r5_pitch<PER>() * 4 > R5_TILE ? R5_ROWS * r5_pitch<PER>() * 4 : R5_TILE;
+}
+
+// A wait that no memory access crosses, in the compiler or the schedule:
+// gfx9 s_waitcnt immediates (vmcnt in bits 3:0 and 15:14, lgkmcnt in 11:8).
+constexpr int WAIT_VM16 = 0x4F70;  // at most 16 vector-memory operations outstanding
+constexpr int WAIT_ALL = 0x0070;   // none, and no LDS or scalar read
+template <int IMM> __device__ __forceinline__ void fence() {
+  __asm__ volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(IMM);
+  __builtin_amdgcn_sched_barrier(0);
+  __asm__ volatile("" ::: "memory");
+}
+
+// Same rows, keys, masks and error flags as decode_generic: the rows of a
+// request's beams in order (row rho: beam rho / (T G), query (rho / G) % T, head
+// rho % G), the keys of a workgroup its request's prefix, then the suffixes of
+// its rows' beams one after another.
+template <int DT, bool SOFTCAP>
+__global__ __launch_bounds__(R5_THREADS) void decode_row512(DecodeArgs a, int units, int chunks) {
+  kernarg_lines<kernarg_line_count<DecodeArgs>(8)>();
+  using E = Elem<DT>;
+  using S = typename E::storage;
+  using M = Row512<DT>;
+  constexpr int PER = M::PER;
+  constexpr int D = 32 * PER;
+  constexpr int REGION = r5_region<PER>();
+  __shared__ __attribute__((aligned(16))) uint8_t tiles[R5_WAVES * REGION];
+  __shared__ int64_t t_off[R5_WAVES][2][R5_KEYS];  // per tile key: element offset of its row, -1: none
+  __shared__ int t_beam[R5_WAVES][2][R5_KEYS];     // ... its chunk beam; -1: a prefix key, -2: no key
+  __shared__ int t_pos[R5_WAVES][2][R5_KEYS];      // ... index in the beam's suffix
+  __shared__ int c_len[R5_ROWS], c_s0[R5_ROWS], c_cum[R5_ROWS + 1];
+  __shared__ float w_m[R5_WAVES][R5_ROWS], w_l[R5_WAVES][R5_ROWS];
+
+  // workgroup -> (request, KV head, row chunk); blockIdx % 8 is the XCD
+  const int seq = blockIdx.x >> 3;
+  const int unit = (seq / chunks) * 8 + (blockIdx.x & 7), chunk = seq % chunks;
+  if (unit >= units) return;
+  const int r = unit / a.Hkv, hk = unit % a.Hkv;
+  const int t = threadIdx.x, lane = t & 63, m16 = lane & 15, qd = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int G = a.Hq / a.Hkv, TG = a.T * G;
+  const int row0 = chunk * R5_ROWS;
+  const int pre_cap = a.prefix_bt_stride * a.bs;
+  const int nb0 = a.beam_start[r];
+  const int W = a.beam_start[r + 1] - nb0;
+  if (nb0 < 0 || W < 0 || nb0 + W > a.num_beams || W > a.max_beams) {
+    if (t == 0 && chunk == 0) flag_status(a.dev_status, GR_DEV_BAD_LENGTH);
+    return;
+  }
+  if (row0 >= W * TG) return;
+  const int nrows = min(R5_ROWS, W * TG - row0);
+  const int P = a.prefix_len[r], Pc = min(max(P, 0), pre_cap);
+  if (t == 0 && chunk == 0 && Pc != P) flag_status(a.dev_status, GR_DEV_BAD_LENGTH);
+  const int b_lo = row0 / TG;
+  const int nbm = (row0 + nrows - 1) / TG - b_lo + 1;  // beams in the chunk (<= 16)
+  if (t < nbm) {
+    const int n = nb0 + b_lo + t;
+    const int L = a.suffix_len[n], s0 = a.suffix_start ? a.suffix_start[n] : 0;
+    const int suf_cap = a.suffix_bt_stride * a.bs;
+    const int Lc = (L < 0 || s0 < 0 || s0 + L > suf_cap) ? 0 : L;
+    if (Lc != L) flag_status(a.dev_status, GR_DEV_BAD_LENGTH);
+    c_len[t] = Lc;
+    c_s0[t] = s0;
+  }
+  __syncthreads();
+  if (t == 0) {
+    int c = 0;
+    for (int j = 0; j < nbm; ++j) {
+      c_cum[j] = c;
+      c += c_len[j];
+    }
+    c_cum[nbm] = c;
+  }
+  __syncthreads();
+  const int total = Pc + c_cum[nbm];
+  const int n_tiles = (total + R5_KEYS - 1) / R5_KEYS;
+
+  const uint8_t* kc = static_cast<const uint8_t*>(a.k_cache) + (int64_t)hk * a.kv_head_stride * (int)sizeof(S);
+  const uint8_t* vc = static_cast<const uint8_t*>(a.v_cache) + (int64_t)hk * a.kv_head_stride * (int)sizeof(S);
+  const uint8_t* zero = reinterpret_cast<const uint8_t*>(g_zero16);
+
+  // this lane's row and its Q: chunks 4 j + g
+  const bool row_ok = m16 < nrows;
+  const int rho = row0 + (row_ok ? m16 : 0);
+  const int my_b = rho / TG - b_lo, my_qi = (rho / G) % a.T, my_g = rho % G;
+  const int64_t my_tok = (int64_t)(nb0 + b_lo + my_b) * a.T + my_qi;
+  const int my_last = c_len[my_b] - a.T + my_qi;  // last suffix index the row sees
+  u32x4_t qf[8];
+  {
+    const uint8_t* qp = static_cast<const uint8_t*>(a.q) +
+                        (my_tok * a.q_tok_stride + (int64_t)(hk * G + my_g) * D) * (int)sizeof(S);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      qf[j] = *reinterpret_cast<const u32x4_t*>(row_ok ? qp + (4 * j + qd) * 16 : zero);
+  }
+
+  // key kk of tile ti (lanes 0 .. 31 one key each): its block id, then its
+  // table entries; the id's load is apart from its use so that it can be in
+  // flight under other work
+  struct KeyRef { int blk, o, beam, pos; };
+  auto key_ref = [&](int ti) {
+    KeyRef k{-1, 0, -2, 0};
+    const int kk = ti * R5_KEYS + lane;
+    if (lane < R5_KEYS && kk < total) {
+      int pos = kk;
+      const int32_t* bt = a.prefix_bt + (int64_t)r * a.prefix_bt_stride;
+      k.beam = -1;
+      if (kk >= Pc) {  // suffix slot j: beam kb holds slots c_cum[kb] .. c_cum[kb + 1] - 1
+        const int j = kk - Pc;
+        int kb = 0;
+        while (c_cum[kb + 1] <= j) ++kb;
+        k.beam = kb;
+        k.pos = j - c_cum[kb];
+        pos = c_s0[kb] + k.pos;
+        bt = a.suffix_bt + (int64_t)(nb0 + b_lo + kb) * a.suffix_bt_stride;
+      }
+      const int bi = a.bs_shift >= 0 ? pos >> a.bs_shift : pos / a.bs;
+      k.o = pos - bi * a.bs;
+      k.blk = bt[bi];
+    }
+    return k;
+  };
+  auto key_store = [&](int buf, const KeyRef& k) {
+    if (lane < R5_KEYS) {
+      const bool ok = k.blk >= 0 && k.blk < a.num_blocks;
+      if (k.beam != -2 && !ok) flag_status(a.dev_status, GR_DEV_BAD_BLOCK);
+      t_off[wave][buf][lane] = ok ? (int64_t)k.blk * a.kv_block_stride + (int64_t)k.o * a.kv_tok_stride : -1;
+      t_beam[wave][buf][lane] = ok ? k.beam : -2;
+      t_pos[wave][buf][lane] = k.pos;
+    }
+  };
+  uint8_t* ktile = tiles + wave * REGION;
+  // tile rows 2 i, 2 i + 1 by load i: position p of row key holds chunk p ^ (key % 16)
+  auto k_load = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < R5_KEYS / 2; ++i) {
+      const int key = 2 * i + (lane >> 5);
+      const int64_t off = t_off[wave][buf][key];
+      const uint8_t* src = off < 0 ? zero : kc + off * (int)sizeof(S) + (((lane & 31) ^ (key & 15)) << 4);
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                       (__attribute__((address_space(3))) void*)(ktile + i * 1024), 16, 0, 0);
+    }
+  };
+
+  f4_t o[2][PER];
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int e = 0; e < PER; ++e) o[c][e] = f4_t{0.f, 0.f, 0.f, 0.f};
+  float mrow = -INFINITY, lsum = 0.f;  // the row's running maximum; this lane's keys' weights
+
+  if (wave < n_tiles) {
+    key_store(0, key_ref(wave));
+    k_load(0);
+  }
+  int buf = 0;
+  for (int ti = wave; ti < n_tiles; ti += R5_WAVES, buf ^= 1) {
+    const bool more = ti + R5_WAVES < n_tiles;
+    const KeyRef nx = key_ref(more ? ti + R5_WAVES : n_tiles);  // (n_tiles: every key past the end)
+    // V rows of this lane's keys: slot 4 kb + r is key 16 kb + 4 g + r
+    u32x4_t vf[2][8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int64_t off = t_off[wave][buf][16 * (s >> 2) + 4 * qd + (s & 3)];
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        vf[c][s] = *reinterpret_cast<const u32x4_t*>(off < 0 ? zero : vc + off * (int)sizeof(S) + (16 * c + m16) * 16);
+    }
+    // This tile's K transfers were issued before the V loads above and return
+    // in order: with at most those 16 outstanding they are in LDS.  (The wait
+    // is written out: the compiler does not order LDS reads after transfers
+    // into LDS in every instantiation.)
+    fence<WAIT_VM16>();
+    f4_t s2[2] = {f4_t{0.f, 0.f, 0.f, 0.f}, f4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        const int key = 16 * kb + m16;
+        const u32x4_t kf = *reinterpret_cast<const u32x4_t*>(ktile + key * R5_BYTES + (((4 * j + qd) ^ m16) << 4));
+        s2[kb] = M::qk(kf, qf[j], s2[kb]);
+      }
+    }
+    // every read of this tile has returned before the next tile lands on it;
+    // V too is waited for here, not behind the next tile's transfers
+    fence<WAIT_ALL>();
+    if (more) {
+      key_store(buf ^ 1, nx);
+      k_load(buf ^ 1);
+    }
+    // online softmax of the lane's 8 scores (row m16; keys 16 kb + 4 g + r)
+    float p[8], mt = -INFINITY;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int key = 16 * (s >> 2) + 4 * qd + (s & 3);
+      float x = s2[s >> 2][s & 3] * a.scale;
+      if constexpr (SOFTCAP) x = a.softcap * tanhf(x / a.softcap);
+      const int kb = t_beam[wave][buf][key], kp = t_pos[wave][buf][key];
+      p[s] = (kb == -1) | ((kb == my_b) & (kp <= my_last)) ? x : -INFINITY;
+      mt = fmaxf(mt, p[s]);
+    }
+    mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    const float mn = fmaxf(mrow, mt);
+    if (__ballot(mn > mrow)) {  // some row's maximum moves: rescale (a row whose own stays multiplies by 1)
+      const float al = mrow == -INFINITY ? 0.f : expf(mrow - mn);
+      lsum *= al;
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int e = 0; e < PER; ++e)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) o[c][e][u] *= al;
+      mrow = mn;
+    }
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      p[s] = p[s] == -INFINITY ? 0.f : expf(p[s] - mrow) * M::PSCALE;
+      lsum += p[s];
+    }
+    if constexpr (DT == GR_DTYPE_F32) {
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int e = 0; e < PER; ++e)
+            o[c][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(vf[c][s][e]), p[s], o[c][e], 0, 0, 0);
+    } else {
+      float hi[8], lo[8];
+#pragma unroll
+      for (int s = 0; s < 8; ++s) M::split(p[s], hi[s], lo[s]);
+      const u32x4_t ph = M::pack(hi), pl = M::pack(lo);
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {  // dims 2 w, 2 w + 1 of the chunk over the 8 keys
+          u32x4_t v0, v1;
+#pragma unroll
+          for (int h = 0; h < 4; ++h) {
+            v0[h] = __builtin_amdgcn_perm(vf[c][2 * h + 1][w], vf[c][2 * h][w], 0x05040100u);
+            v1[h] = __builtin_amdgcn_perm(vf[c][2 * h + 1][w], vf[c][2 * h][w], 0x07060302u);
+          }
+          o[c][2 * w] = M::mma(v0, ph, o[c][2 * w]);
+          o[c][2 * w + 1] = M::mma(v1, ph, o[c][2 * w + 1]);
+          o[c][2 * w] = M::mma(v0, pl, o[c][2 * w]);
+          o[c][2 * w + 1] = M::mma(v1, pl, o[c][2 * w + 1]);
+        }
+    }
+  }
+
+  // ---- merge of the waves' states, in LDS ------------------------------------
+  lsum += __shfl_xor(lsum, 16, 64);
+  lsum += __shfl_xor(lsum, 32, 64);
+  if (qd == 0) {
+    w_m[wave][m16] = mrow;
+    w_l[wave][m16] = lsum;
+  }
+  __syncthreads();
+  // a sink joins the row's softmax: in the maximum and, once, in the sum
+  auto row_max = [&](int row, float sink) {
+    float m = sink;
+#pragma unroll
+    for (int w = 0; w < R5_WAVES; ++w) m = fmaxf(m, w_m[w][row]);
+    return m;
+  };
+  {
+    const float sink = a.sinks ? a.sinks[hk * G + my_g] : -INFINITY;
+    const float m = row_max(m16, sink);
+    const float f = mrow == -INFINITY ? 0.f : expf(mrow - m);
+    // accumulator (c, e), register u of quarter g: dim PER (16 c + 4 g + u) + e
+    float* po = reinterpret_cast<float*>(tiles + wave * REGION) + m16 * r5_pitch<PER>();
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int e = 0; e < PER; e += 4)
+          *reinterpret_cast<f4_t*>(po + PER * (16 * c + 4 * qd + u) + e) =
+              f4_t{o[c][e][u] * f, o[c][e + 1][u] * f, o[c][e + 2][u] * f, o[c][e + 3][u] * f};
+  }
+  __syncthreads();
+  // one thread per (row, 16-byte chunk of the output)
+  const int orow = t >> 5, och = t & 31;
+  static_assert(R5_ROWS * 32 == R5_THREADS, "a thread per output chunk");
+  if (orow >= nrows) return;
+  const int orho = row0 + orow;
+  const int og = orho % G;
+  const int64_t otok = (int64_t)(nb0 + orho / TG) * a.T + (orho / G) % a.T;
+  const float sink = a.sinks ? a.sinks[hk * G + og] : -INFINITY;
+  const float m = row_max(orow, sink);
+  float l = 0.f;
+#pragma unroll
+  for (int w = 0; w < R5_WAVES; ++w) {
+    const float mw = w_m[w][orow];
+    if (mw != -INFINITY) l += w_l[w][orow] * expf(mw - m);
+  }
+  l *= 1.f / M::PSCALE;
+  if (sink != -INFINITY) l += expf(sink - m);
+  float v[PER];
+#pragma unroll
+  for (int e = 0; e < PER; ++e) v[e] = 0.f;
+#pragma unroll
+  for (int w = 0; w < R5_WAVES; ++w) {
+    const float* po = reinterpret_cast<const float*>(tiles + w * REGION) + orow * r5_pitch<PER>() + PER * och;
+#pragma unroll
+    for (int e = 0; e < PER; e += 4) {
+      const f4_t x = *reinterpret_cast<const f4_t*>(po + e);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[e + u] += x[u];
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < PER; ++e) v[e] = l > 0.f ? v[e] * (1.f / M::PSCALE) / l : 0.f;
+  *reinterpret_cast<u32x4_t*>(static_cast<S*>(a.out) + otok * a.out_tok_stride + (int64_t)(hk * G + og) * D + PER * och) =
+      M::pack(v);
+  if (a.lse_out && och == 0) a.lse_out[otok * a.Hq + hk * G + og] = l > 0.f ? m + logf(l) : -INFINITY;
+}
+
+}  // namespace
+
+// Plain, soft-capped and sink decodes whose rows are 512 bytes and 16-byte
+// aligned throughout (bases and strides in whole chunks).  Windows, ALiBi and
+// fp8 caches stay on the generic kernel.
+bool row512_decode_supported(const DecodeArgs& a) {
+  const int es = dtype_size(a.dtype);
+  if (a.D * es != R5_BYTES || a.kv8 || a.alibi || a.win_left >= 0 || a.win_right >= 0 || !a.causal) return false;
+  if (a.num_blocks < 1) return false;
+  auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  if (!al(a.q) || !al(a.out) || !al(a.k_cache) || !al(a.v_cache)) return false;
+  const int ch = 16 / es;
+  if (a.q_tok_stride % ch || a.out_tok_stride % ch || a.kv_block_stride % ch || a.kv_tok_stride % ch ||
+      a.kv_head_stride % ch)
+    return false;
+  return true;
+}
+
+gr_status_t launch_row512_decode(const DecodeArgs& a, hipStream_t stream) {
+  const int64_t rows = (int64_t)a.max_beams * a.T * (a.Hq / a.Hkv);
+  const int64_t ch64 = (rows + R5_ROWS - 1) / R5_ROWS;
+  const int64_t units64 = (int64_t)a.num_reqs * a.Hkv;
+  if (ch64 == 0 || units64 == 0) return GR_OK;
+  const int64_t nwg = (units64 + 7) / 8 * 8 * ch64;
+  if (nwg > 0x7fffffff) return GR_ERR_INVALID_ARG;
+  const int units = (int)units64, chunks = (int)ch64;
+  const dim3 grid((unsigned)nwg), blk(R5_THREADS);
+  const bool cap = a.softcap > 0.f;
+#define GR_ROW512(DT)                                                                                       \
+  do {                                                                                                      \
+    if (cap) hipLaunchKernelGGL((decode_row512<DT, true>), grid, blk, 0, stream, a, units, chunks);         \
+    else hipLaunchKernelGGL((decode_row512<DT, false>), grid, blk, 0, stream, a, units, chunks);            \
+  } while (0)
+  if (a.dtype == GR_DTYPE_F32) GR_ROW512(GR_DTYPE_F32);
+  else if (a.dtype == GR_DTYPE_F16) GR_ROW512(GR_DTYPE_F16);
+  else GR_ROW512(GR_DTYPE_BF16);
+#undef GR_ROW512
+  return launch_status();
+}
+
+}  // namespace gr
