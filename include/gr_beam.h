@@ -350,6 +350,14 @@ gr_status_t gr_beam_kv_append(
 size_t gr_beam_prune_workspace_size(int num_reqs, int beam_width, int vocab, int k);
 
 /*
+ * The workspace with which long rows (k <= 256) run fastest: the
+ * base size plus room for partial results, so that several workgroups share a
+ * row.  Never less than gr_beam_prune_workspace_size(), which stays enough for
+ * every call; the results are the same bit for bit.
+ */
+size_t gr_beam_prune_workspace_size_split(int num_reqs, int beam_width, int vocab, int k);
+
+/*
  * gr_beam_prune_topk constrained by a catalog of valid semantic-ID token
  * sequences (the reference's Catalog trie, vllm_gr/entrypoints/openai/
  * serving_models.py:18-49, applied at serving_engine.py:381-394, 504-506,

@@ -1,0 +1,75 @@
+"""Pruning of long rows (from 20480 logits) over several workgroups a row, bit for bit
+against the CPU oracle, at the edges of its range and of its chunks (1024 logits), slices and
+72-chunk panels; and the same bits from the base workspace (one workgroup a row)."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import prune as op
+from vllm_gr_amd import _C, ops, workloads
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(t):
+    a = t.cpu().numpy()
+    return a.view({4: np.int32, 8: np.int64}[a.itemsize])
+
+
+def _run(wl, device, eos=-1, base=False):
+    d = wl.to(device)
+    R, W, V = wl.logits.shape
+    n = (_C.lib().gr_beam_prune_workspace_size if base else _C.lib().gr_beam_prune_workspace_size_split)(R, W, V, wl.k)
+    # garbage in the workspace: nothing may be taken from it before it is written
+    ws = torch.full((n,), 0xA5, dtype=torch.uint8, device=device)
+    out = ops.beam_prune_topk(d.logits, d.cum, wl.k, eos, workspace=ws)
+    torch.cuda.synchronize()
+    return out
+
+
+def _check(wl, device, eos=-1):
+    want = op.prune_topk(wl.logits.numpy(), wl.cum.numpy(), wl.k, eos)
+    got = _run(wl, device, eos)
+    for g, name in zip(got, ("parent", "token", "score", "eos_score")):
+        assert np.array_equal(_bits(g), want[name].view(np.int32)), name
+    for g, b in zip(got, _run(wl, device, eos, base=True)):
+        assert np.array_equal(_bits(g), _bits(b))
+
+
+@pytest.mark.parametrize("R,W,V,k", [(1, 1, 20476, 9), (1, 1, 20480, 1), (2, 3, 20484, 256), (1, 5, 21504, 100), (2, 2, 65536, 32),
+                                     (1, 2, 73728, 17), (1, 3, 73732, 64), (1, 4, 151936, 32), (3, 4, 22528, 300), (2, 300, 32768, 8)])
+def test_split_rows(device, R, W, V, k):
+    _check(workloads.make_prune(R=R, W=W, V=V, k=k, seed=V + k), device)
+
+
+@pytest.mark.parametrize("kind", ["ties", "equal", "masked", "tail", "eos"])
+def test_split_rows_hard_inputs(device, kind):
+    """Many ties at the bound, one value throughout (more survivors than the
+    list holds), masked tokens and a masked beam, the best at the row's end, EOS."""
+    wl = workloads.make_prune(R=2, W=4, V=20488, k=32, seed=3)
+    lg = wl.logits
+    if kind == "ties":
+        lg.copy_(torch.round(lg))
+    elif kind == "equal":
+        lg.fill_(1.5)
+        lg[0, 0] = -0.0
+    elif kind == "masked":
+        lg[0, :, 10:] = float("-inf")
+        lg[1, 2] = float("-inf")
+    elif kind == "tail":
+        lg[:, :, -40:] += 50.0
+    _check(wl, device, eos=int(lg[0, 0].argmax()) if kind == "eos" else -1)
+
+
+def test_split_rows_f64_lists(device):
+    """float64 scores and the candidate lists: the same bits from either workspace."""
+    wl = workloads.make_prune(R=2, W=8, V=40004, k=48, seed=9)
+    lg, cum = wl.logits.to(device), wl.cum.to(device).double()
+    res = []
+    for size in (_C.lib().gr_beam_prune_workspace_size, _C.lib().gr_beam_prune_workspace_size_split):
+        ws = torch.empty(size(2, 8, 40004, 48), dtype=torch.uint8, device=device)
+        res.append(ops.beam_prune_topk(lg, cum, 48, 5, workspace=ws, candidates=True))
+    torch.cuda.synchronize()
+    for x, y in zip(*res):
+        assert np.array_equal(_bits(x), _bits(y))

@@ -125,6 +125,13 @@ struct PruneArgs {
   uint64_t* part_key;  // [R, ng, k] stage-1 selections: score key (0 = empty) ...
   int64_t* part_flat;  // ... and flat index b * V + v
   int ng, gr;          // row groups per request, rows per group
+  // long rows split over workgroups (prune_slice_max / prune_slice_sum), per row:
+  float* sl_max;       // [SL_MAX] maxima of disjoint parts of the row
+  float* sl_acc;       // [PR_THREADS] exp-sum partials in prune_rows' thread order
+  uint64_t* sl_surv;   // [PR_SURV] survivors: (logit bits, token)
+  int32_t* sl_n;       // survivors found (may exceed PR_SURV)
+  float* sl_m;         // the row's maximum
+  uint32_t* sl_t0;     // the survivors' bound as a key
   // catalog (nullable): the trie in CSR form -- node n's children are
   // child_token / child_node[node_start[n] .. node_start[n+1]), tokens
   // ascending; beam_node[b] is beam b's node (-1: no valid continuation)
@@ -389,6 +396,194 @@ __device__ __noinline__ void row_topk_radix(const float* xg, int V, int k1, uint
   }
 }
 
+// ---- rows past the register-resident size, split over workgroups ------------
+// One workgroup per row walks a long row four times (maximum, sum, survivor
+// count, survivors) in PR_CHUNK steps with one wave of loads in flight: 250 us
+// for 128 rows of 151936, 0.3 TB/s, half of the chip idle.  Two short launches
+// over SL_NS workgroups per row read it twice instead: the maxima of 2048
+// disjoint parts, then (with the row's maximum and the selection bound that
+// these give) the exponentials and the survivors.  prune_rows<SPLIT> goes on
+// from there.  128 rows of 151936: 250 -> 13.4 (5.8 TB/s) + 24.7 + 4.6 us.
+//
+// The fixed summation order is prune_rows': logical thread c of 256 adds the
+// elements 4 c .. 4 c + 3 of every chunk in turn.  Slice s holds the logical
+// threads 32 s .. 32 s + 31 -- 512 contiguous bytes of each chunk -- and its
+// 256 threads work out eight chunks' exponentials side by side into LDS, where
+// 32 threads then add them in order: every partial is the same float.
+constexpr int SL_NS = 8;                              // workgroups per row
+constexpr int SL_COLS = PR_THREADS / SL_NS;           // logical threads per slice
+constexpr int SL_SIDE = PR_THREADS / SL_COLS;         // chunks side by side
+constexpr int SL_STEPS = 9;                           // loads in flight per thread
+constexpr int SL_PANEL = SL_SIDE * SL_STEPS;          // chunks per LDS panel (36 KB; with the list 40 KB: four workgroups a CU)
+constexpr int SL_LIST = PR_SURV - 2;                  // survivors a slice holds (its counter takes the rest)
+constexpr int SL_MAX = SL_NS * PR_THREADS;            // part maxima per row
+
+__global__ __launch_bounds__(PR_THREADS) void prune_slice_max(PruneArgs a) {
+  const int row = blockIdx.x / SL_NS, slice = blockIdx.x % SL_NS, tid = threadIdx.x;
+  const float* xg = a.logits + (int64_t)row * a.row_stride;
+  const int V = a.V, col = 4 * (slice * SL_COLS + tid % SL_COLS);
+  // every part holds an element: V > 8 chunks
+  float m = -INFINITY;
+  int c = tid / SL_COLS;
+  for (; (int64_t)(c + 7 * SL_SIDE + 1) * PR_CHUNK <= V; c += 8 * SL_SIDE) {  // eight whole chunks, loads together
+    f32x4_t v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      v[i] = *reinterpret_cast<const f32x4_t*>(xg + (int64_t)(c + i * SL_SIDE) * PR_CHUNK + col);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m = fmaxf(m, fmaxf(fmaxf(v[i][0], v[i][1]), fmaxf(v[i][2], v[i][3])));
+  }
+#pragma unroll 4
+  for (; (int64_t)c * PR_CHUNK + col < V; c += SL_SIDE) {
+    const f32x4_t v = *reinterpret_cast<const f32x4_t*>(xg + (int64_t)c * PR_CHUNK + col);
+    m = fmaxf(m, fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])));
+  }
+  a.sl_max[(int64_t)row * SL_MAX + slice * PR_THREADS + tid] = m;
+  if (slice == 0 && tid == 0) a.sl_n[row] = 0;
+}
+
+__global__ __launch_bounds__(PR_THREADS) void prune_slice_sum(PruneArgs a) {
+  __shared__ f32x4_t ex[SL_PANEL * SL_COLS];
+  // (in the panel's space, which is written after they are read)
+  float* wred = reinterpret_cast<float*>(ex);
+  uint32_t* wkey = reinterpret_cast<uint32_t*>(ex) + PR_THREADS / 64;
+  // the slice's survivors: one atomic per slice on the row's counter (per wave
+  // and step, its round trips were most of this kernel's time)
+  __shared__ struct { uint64_t raw[SL_LIST]; int n; } list;
+  const int row = blockIdx.x / SL_NS, slice = blockIdx.x % SL_NS;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const float* xg = a.logits + (int64_t)row * a.row_stride;
+  const int V = a.V, k1 = a.k1;
+  const int nch = (V + PR_CHUNK - 1) / PR_CHUNK;
+  const int col = 4 * (slice * SL_COLS + tid % SL_COLS), c0 = tid / SL_COLS;
+  const int own = (V - col - 1) / PR_CHUNK + 1;  // chunks in which this column has elements
+  // equal panels of whole side-by-side steps
+  const int np = (nch + SL_PANEL - 1) / SL_PANEL;
+  const int per = ((nch + np - 1) / np + SL_SIDE - 1) / SL_SIDE * SL_SIDE;
+  // a panel's loads, all in flight at once; the first panel's under the bound
+  // search, the others' under the previous panel's ordered additions
+  f32x4_t v[SL_STEPS];
+  auto load = [&](int p0) {
+#pragma unroll
+    for (int i = 0; i < SL_STEPS; ++i) {
+      const int c = p0 + c0 + i * SL_SIDE;
+      if (i * SL_SIDE < per)
+        v[i] = *reinterpret_cast<const f32x4_t*>(xg + (c < own ? (int64_t)c * PR_CHUNK + col : 0));
+    }
+  };
+  load(0);
+  // row maximum and bound t0 from the 2048 part maxima, eight a lane: per wave
+  // the ceil(k1 / 4)-th largest of its 512, rounded down to the key's top 16
+  // bits, least over the waves (the maxima are distinct elements, so at least
+  // k1 keys are >= t0)
+  constexpr int MPL = SL_MAX / PR_THREADS;
+  float pm[MPL];
+  {
+    const f32x4_t* pp = reinterpret_cast<const f32x4_t*>(a.sl_max + (int64_t)row * SL_MAX) + tid;
+#pragma unroll
+    for (int i = 0; i < MPL / 4; ++i) {
+      const f32x4_t v = pp[i * PR_THREADS];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) pm[4 * i + j] = v[j] + 0.0f;
+    }
+  }
+  float tm = pm[0];
+#pragma unroll
+  for (int i = 1; i < MPL; ++i) tm = fmaxf(tm, pm[i]);
+  const float wm = wave_max(tm);
+  if (lane == 0) wred[wave] = wm;
+  __syncthreads();
+  float m = wred[0];
+#pragma unroll
+  for (int w = 1; w < PR_THREADS / 64; ++w) m = fmaxf(m, wred[w]);
+  {
+    const int kw = (k1 + 3) >> 2;
+    uint32_t ak[MPL];
+#pragma unroll
+    for (int i = 0; i < MPL; ++i) ak[i] = fkey(pm[i]) >> 16;
+    uint32_t lo = 0, hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(fkey(m) >> 16));
+    auto count_ge = [&](uint32_t v) {
+      int n = 0;
+#pragma unroll
+      for (int i = 0; i < MPL; ++i) n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(ak[i] >= v));
+      return n;
+    };
+    if (hi > 256 && count_ge(hi - 256) >= kw) lo = hi - 256;
+    while (lo < hi) {
+      const uint32_t mid = lo + ((hi - lo + 1) >> 1);
+      if (count_ge(mid) >= kw) lo = mid;
+      else hi = mid - 1;
+    }
+    if (lane == 0) wkey[wave] = lo << 16;
+  }
+  __syncthreads();
+  uint32_t t0 = wkey[0];
+#pragma unroll
+  for (int w = 1; w < PR_THREADS / 64; ++w) t0 = min(t0, wkey[w]);
+  if (t0 <= fkey(-INFINITY)) t0 = 0;
+  const float t0f = t0 == 0 ? -INFINITY : fval(t0);
+  if (slice == 0 && tid == 0) {
+    a.sl_m[row] = m;
+    a.sl_t0[row] = t0;
+  }
+
+  const float ml = m * 0x1.715476p+0f;
+  float acc = 0.0f;
+  if (tid == 0) list.n = 0;
+  __syncthreads();  // wred and wkey are read
+  for (int p0 = 0; p0 < nch; p0 += per) {
+#pragma unroll
+    for (int i = 0; i < SL_STEPS; ++i) {
+      if (i * SL_SIDE >= per) break;
+      const int c = p0 + c0 + i * SL_SIDE;
+      const bool in = c < own;
+      f32x4_t e;
+      int ns = 0;
+#pragma unroll
+      for (int j = 0; j < PR_VEC; ++j) {
+        const float y = v[i][j] + 0.0f;
+        const float t = __builtin_fmaf(y, 0x1.715476p+0f, -ml);
+        e[j] = exp2_neg(t);
+        ns += in & (y >= t0f);
+      }
+      ex[(c0 + i * SL_SIDE) * SL_COLS + tid % SL_COLS] = e;
+      if (ns != 0) {
+        int pos = atomicAdd(&list.n, ns);
+#pragma unroll
+        for (int j = 0; j < PR_VEC; ++j) {
+          const float y = v[i][j] + 0.0f;
+          if (y >= t0f) {
+            if (pos < SL_LIST)
+              list.raw[pos] = ((uint64_t)__builtin_bit_cast(uint32_t, y) << 32) | (uint32_t)(c * PR_CHUNK + col + j);
+            ++pos;
+          }
+        }
+      }
+    }
+    if (p0 + per < nch) load(p0 + per);
+    __syncthreads();
+    if (tid < SL_COLS) {
+      const int n = min(own - p0, per);
+#pragma unroll 8
+      for (int c = 0; c < n; ++c) {
+        const f32x4_t e = ex[c * SL_COLS + tid];
+#pragma unroll
+        for (int j = 0; j < PR_VEC; ++j) acc = acc + e[j];
+      }
+    } else if (wave == 1 && p0 + per >= nch) {  // the list is complete
+      const int n = list.n;
+      int base = 0;
+      // (a list that overflowed sends the row to the radix path, whatever the other slices hold)
+      if (lane == 0 && n > 0) base = atomicAdd(&a.sl_n[row], n <= SL_LIST ? n : PR_SURV + 1);
+      base = __builtin_amdgcn_readfirstlane(base);
+      for (int i = lane; i < min(n, SL_LIST); i += 64)
+        if (base + i < PR_SURV) a.sl_surv[(int64_t)row * PR_SURV + base + i] = list.raw[i];
+    }
+    __syncthreads();
+  }
+  if (tid < SL_COLS) a.sl_acc[(int64_t)row * PR_THREADS + slice * SL_COLS + tid] = acc;
+}
+
 // MAXC > 0: row held in registers (<= MAXC chunks); 0: re-read from memory.
 // CATALOG: the beam's top-k candidates outside its trie node's children are
 // dropped (the reference masks them to -inf after the sampler's per-beam
@@ -396,7 +591,9 @@ __device__ __noinline__ void row_topk_radix(const float* xg, int V, int k1, uint
 // FULL: the row is exactly MAXC chunks (V = MAXC * PR_CHUNK), so every chunk
 // and element is live: no padding, no per-chunk bounds tests (the same
 // arithmetic, in the same order, as the general form).
-template <int MAXC, bool CATALOG = false, bool FULL = false>
+// SPLIT: maximum, exp-sum partials, bound and survivors come from the slice
+// kernels.
+template <int MAXC, bool CATALOG = false, bool FULL = false, bool SPLIT = false>
 __global__ __launch_bounds__(PR_THREADS) void prune_rows(PruneArgs a) {
   static_assert(!FULL || MAXC > 0, "a full row is held in registers");
   __shared__ uint64_t sk[PR_MAXK];  // candidates as row_key
@@ -455,34 +652,42 @@ __global__ __launch_bounds__(PR_THREADS) void prune_rows(PruneArgs a) {
 
   // ---- row max; also the thread's second-largest chunk maximum (an element
   // other than the thread maximum: it tightens the selection bound below) ----
-  float tm = -INFINITY, t2 = -INFINITY;
-  PR_FOR_CHUNKS(c) {
-    if (live(c)) {
-      const float cm = fmaxf(fmaxf(get(c, 0), get(c, 1)), fmaxf(get(c, 2), get(c, 3)));
-      t2 = fmaxf(t2, cm >= tm ? tm : cm);  // NaN chunk maxima (all four NaN) are skipped
-      tm = fmaxf(tm, cm);
+  float tm = -INFINITY, t2 = -INFINITY, m;
+  if constexpr (SPLIT) {
+    m = a.sl_m[row];
+  } else {
+    PR_FOR_CHUNKS(c) {
+      if (live(c)) {
+        const float cm = fmaxf(fmaxf(get(c, 0), get(c, 1)), fmaxf(get(c, 2), get(c, 3)));
+        t2 = fmaxf(t2, cm >= tm ? tm : cm);  // NaN chunk maxima (all four NaN) are skipped
+        tm = fmaxf(tm, cm);
+      }
     }
-  }
-  const float wm = wave_max(tm);
-  if (lane == 0) wred[wave] = wm;
-  __syncthreads();
-  float m = wred[0];
+    const float wm = wave_max(tm);
+    if (lane == 0) wred[wave] = wm;
+    __syncthreads();
+    m = wred[0];
 #pragma unroll
-  for (int w = 1; w < PR_THREADS / 64; ++w) m = fmaxf(m, wred[w]);
-  __syncthreads();
+    for (int w = 1; w < PR_THREADS / 64; ++w) m = fmaxf(m, wred[w]);
+    __syncthreads();
+  }
 
   // ---- fixed-order exp-sum: thread partial in element order, xor butterfly, waves pairwise ----
   double c_row = -INFINITY;
   double lse_row = INFINITY;  // a row of -inf logits has logprobs -inf
   if (m != -INFINITY) {
     float acc = 0.0f;
-    const float ml = m * 0x1.715476p+0f;
-    PR_FOR_CHUNKS(c) {
-      if (live(c)) {
+    if constexpr (SPLIT) {
+      acc = a.sl_acc[(int64_t)row * PR_THREADS + tid];
+    } else {
+      const float ml = m * 0x1.715476p+0f;
+      PR_FOR_CHUNKS(c) {
+        if (live(c)) {
 #pragma unroll
-        for (int j = 0; j < PR_VEC; ++j) {
-          const float t = __builtin_fmaf(get(c, j), 0x1.715476p+0f, -ml);
-          acc = acc + exp2_neg(t);
+          for (int j = 0; j < PR_VEC; ++j) {
+            const float t = __builtin_fmaf(get(c, j), 0x1.715476p+0f, -ml);
+            acc = acc + exp2_neg(t);
+          }
         }
       }
     }
@@ -508,7 +713,9 @@ __global__ __launch_bounds__(PR_THREADS) void prune_rows(PruneArgs a) {
   // all.  Only keys >= t0 can be selected; with few of them they are ranked
   // directly.
   uint32_t t0 = 0;
-  if (k1 <= PR_THREADS) {
+  if constexpr (SPLIT) {
+    t0 = a.sl_t0[row];
+  } else if (k1 <= PR_THREADS) {
     const int kw = (k1 + 3) >> 2;
     const uint32_t a0 = fkey(tm) >> 16;  // the top 16 bits of the key suffice for a bound
     const uint32_t a1 = fkey(t2) >> 16;
@@ -537,30 +744,37 @@ __global__ __launch_bounds__(PR_THREADS) void prune_rows(PruneArgs a) {
     // patterns 0 .. fkey(-inf)) admits every key
     if (t0 <= fkey(-INFINITY)) t0 = 0;
   }
-  // the same bound on the logits (t0 = 0 admits every key)
-  const float t0f = t0 == 0 ? -INFINITY : fval(t0);
-  // survivors -> LDS in thread order (a block scan hands out each thread's slots)
-  int ns = 0;
-  PR_FOR_CHUNKS(c) {
-    if (live(c)) {
-#pragma unroll
-      for (int j = 0; j < PR_VEC; ++j) ns += get(c, j) >= t0f;
-    }
-  }
-  int pos;
-  // (the total is the same in every thread: held in a scalar register)
-  const int n_surv = __builtin_amdgcn_readfirstlane(block_scan(ns, pos, itmp));
-  // more than PR_SURV survivors: the radix path below selects from the row
-  // itself, so nothing is written (and no write needs a bound check)
-  if (n_surv <= PR_SURV && ns > 0) {
+  int n_surv;
+  if constexpr (SPLIT) {
+    n_surv = __builtin_amdgcn_readfirstlane(a.sl_n[row]);
+    if (n_surv <= PR_SURV)
+      for (int i = tid; i < n_surv; i += PR_THREADS) sk[i] = a.sl_surv[(int64_t)row * PR_SURV + i];
+  } else {
+    // the same bound on the logits (t0 = 0 admits every key)
+    const float t0f = t0 == 0 ? -INFINITY : fval(t0);
+    // survivors -> LDS in thread order (a block scan hands out each thread's slots)
+    int ns = 0;
     PR_FOR_CHUNKS(c) {
       if (live(c)) {
 #pragma unroll
-        for (int j = 0; j < PR_VEC; ++j) {
-          const float y = get(c, j);
-          if (y >= t0f) {  // (logit bits, token); made a row key once, below
-            sk[pos] = ((uint64_t)__builtin_bit_cast(uint32_t, y) << 32) | (uint32_t)(c * PR_CHUNK + PR_VEC * tid + j);
-            ++pos;
+        for (int j = 0; j < PR_VEC; ++j) ns += get(c, j) >= t0f;
+      }
+    }
+    int pos;
+    // (the total is the same in every thread: held in a scalar register)
+    n_surv = __builtin_amdgcn_readfirstlane(block_scan(ns, pos, itmp));
+    // more than PR_SURV survivors: the radix path below selects from the row
+    // itself, so nothing is written (and no write needs a bound check)
+    if (n_surv <= PR_SURV && ns > 0) {
+      PR_FOR_CHUNKS(c) {
+        if (live(c)) {
+#pragma unroll
+          for (int j = 0; j < PR_VEC; ++j) {
+            const float y = get(c, j);
+            if (y >= t0f) {  // (logit bits, token); made a row key once, below
+              sk[pos] = ((uint64_t)__builtin_bit_cast(uint32_t, y) << 32) | (uint32_t)(c * PR_CHUNK + PR_VEC * tid + j);
+              ++pos;
+            }
           }
         }
       }
@@ -1473,6 +1687,28 @@ extern "C" size_t gr_beam_prune_workspace_size(int num_reqs, int beam_width, int
          align256(rows * sizeof(double)) + align256(parts * sizeof(uint64_t)) + align256(parts * sizeof(int64_t));
 }
 
+// Rows that the split path takes (k1 survivors are ranked directly), and its
+// workspace past the base's.  Its two launches and their bound search cost
+// about 15 us, and as much again for every 1024 workgroups, so it waits for
+// rows long enough to be worth it.  Whole call, one workgroup a row -> split:
+// 128 rows of 16384 31.2 -> 29.8 us, 24576 39.3 -> 30.3, 32000 46.5 -> 31.1,
+// 65536 76.6 -> 34.9, 151936 259 -> 52; 4 rows of 16384 27.7 -> 28.4; 256 rows
+// of 32000 64 -> 42; 1024 rows of 32000 108.5 -> 107.4, 65536 195 -> 146; 4096
+// rows of 65536 815 -> 515.
+static bool split_rows(size_t rows, int vocab, int k) {
+  return vocab >= (rows <= 256 ? 20480 : 32768) && k <= PR_THREADS;
+}
+static size_t split_bytes(size_t rows) {
+  return align256(rows * SL_MAX * sizeof(float)) + align256(rows * PR_THREADS * sizeof(float)) +
+         align256(rows * PR_SURV * sizeof(uint64_t)) + 3 * align256(rows * sizeof(int32_t));
+}
+
+extern "C" size_t gr_beam_prune_workspace_size_split(int num_reqs, int beam_width, int vocab, int k) {
+  const size_t base = gr_beam_prune_workspace_size(num_reqs, beam_width, vocab, k);
+  if (base == 0 || !split_rows((size_t)num_reqs * beam_width, vocab, k)) return base;
+  return base + split_bytes((size_t)num_reqs * beam_width);
+}
+
 // The new beam's trie node: the child of its parent's node reached by its
 // token (a selected candidate is always such a child).
 __global__ void catalog_advance(PruneArgs a, int32_t* node_out) {
@@ -1528,7 +1764,28 @@ static gr_status_t prune_launch(PruneArgs& a, const float* logits, int64_t logit
   a.part_key = reinterpret_cast<uint64_t*>(part_base);
   a.part_flat = reinterpret_cast<int64_t*>(part_base + align256(parts * sizeof(uint64_t)));
   const bool cat = a.beam_node != nullptr;
-  if (vocab == PR_CHUNK * PR_REG_CHUNKS) {
+  // Long rows go over several workgroups each where the workspace has the room
+  // (gr_beam_prune_workspace_size_split).
+  const bool split = split_rows(rows, vocab, k) && workspace_bytes >= need + split_bytes(rows) &&
+                     rows * SL_NS <= 0x7fffffff;
+  if (split) {
+    uint8_t* p = ws + need;
+    a.sl_max = reinterpret_cast<float*>(p);
+    p += align256(rows * SL_MAX * sizeof(float));
+    a.sl_acc = reinterpret_cast<float*>(p);
+    p += align256(rows * PR_THREADS * sizeof(float));
+    a.sl_surv = reinterpret_cast<uint64_t*>(p);
+    p += align256(rows * PR_SURV * sizeof(uint64_t));
+    a.sl_n = reinterpret_cast<int32_t*>(p);
+    p += align256(rows * sizeof(int32_t));
+    a.sl_m = reinterpret_cast<float*>(p);
+    p += align256(rows * sizeof(float));
+    a.sl_t0 = reinterpret_cast<uint32_t*>(p);
+    hipLaunchKernelGGL(prune_slice_max, dim3((unsigned)(rows * SL_NS)), dim3(PR_THREADS), 0, stream, a);
+    hipLaunchKernelGGL(prune_slice_sum, dim3((unsigned)(rows * SL_NS)), dim3(PR_THREADS), 0, stream, a);
+    if (cat) hipLaunchKernelGGL((prune_rows<0, true, false, true>), dim3((unsigned)rows), dim3(PR_THREADS), 0, stream, a);
+    else hipLaunchKernelGGL((prune_rows<0, false, false, true>), dim3((unsigned)rows), dim3(PR_THREADS), 0, stream, a);
+  } else if (vocab == PR_CHUNK * PR_REG_CHUNKS) {
     if (cat) hipLaunchKernelGGL((prune_rows<PR_REG_CHUNKS, true, true>), dim3((unsigned)rows), dim3(PR_THREADS), 0, stream, a);
     else hipLaunchKernelGGL((prune_rows<PR_REG_CHUNKS, false, true>), dim3((unsigned)rows), dim3(PR_THREADS), 0, stream, a);
   } else if (vocab <= PR_CHUNK * PR_REG_CHUNKS) {

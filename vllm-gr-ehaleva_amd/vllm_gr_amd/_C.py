@@ -118,6 +118,7 @@ SIGNATURES = {
         _P, _P, _L, _P, _P, _L, _L, _L, _L, _P, _I, _P, _I, _I, _I, _I, _I, _P, _P,
     ]),
     "gr_beam_prune_workspace_size": (_SZ, [_I, _I, _I, _I]),
+    "gr_beam_prune_workspace_size_split": (_SZ, [_I, _I, _I, _I]),
     "gr_beam_prune_topk_catalog": (_I, [
         _P, _L, _P, _I, _I, _I, _I, _I,    # logits, stride, cum, R, W, V, k, eos
         _P, _P, _P, _P, _I, _I,            # beam_node, node_start, child_token, child_node, nodes, edges

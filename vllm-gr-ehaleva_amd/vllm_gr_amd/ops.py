@@ -479,7 +479,9 @@ def beam_kv_append(k_new: torch.Tensor, v_new: torch.Tensor, k_cache: torch.Tens
 
 
 def prune_workspace_bytes(num_reqs: int, beam_width: int, vocab: int, k: int) -> int:
-    return int(_C.lib().gr_beam_prune_workspace_size(num_reqs, beam_width, vocab, k))
+    """Workspace of ``beam_prune_topk``, with the room that long rows use
+    (``gr_beam_prune_workspace_size`` bytes are always enough)."""
+    return int(_C.lib().gr_beam_prune_workspace_size_split(num_reqs, beam_width, vocab, k))
 
 
 def beam_prune_topk(logits: torch.Tensor, cum: torch.Tensor, k: int, eos_token_id: int = -1, *,
@@ -587,7 +589,7 @@ def beam_prune_topk_noalloc(logits: torch.Tensor, cum: torch.Tensor, k: int, eos
     parent, token, score, eos_score = out
     if parent.shape != (R, k) or token.shape != (R, k) or score.shape != (R, k) or eos_score.shape != (R, W):
         raise ValueError("out must be (parent [R,k], token [R,k], score [R,k], eos_score [R,W])")
-    need = prune_workspace_bytes(R, W, V, k)
+    need = int(_C.lib().gr_beam_prune_workspace_size(R, W, V, k))
     if need > _C.GR_PRUNE_SCRATCH_BYTES:
         raise ValueError(f"gr_beam_prune_topk_noalloc: this call needs {need} bytes of scratch; the static "
                          f"scratch holds {_C.GR_PRUNE_SCRATCH_BYTES} (use beam_prune_topk with a workspace)")
