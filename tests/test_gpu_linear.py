@@ -1,0 +1,50 @@
+"""gr_linear against float64 at the edges of its tiles (64 x 64 to 128 x 192), of
+its pipeline (8 stages of 64 features and more) and of its fragments (16
+columns).
+
+Bounds: float32 sums of K products differ from the exact sum by at most K 2^-24
+of the sum of their magnitudes (here taken with a factor of 1/8: errors of both
+signs); a 16-bit output adds half a unit in the last place (2^-8 bf16, 2^-11
+fp16), and SwiGLU's exponential and quotient a few float32 units."""
+
+import pytest
+import torch
+
+from vllm_gr_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 512), (5, 48, 576), (64, 64, 640), (65, 80, 1024), (127, 208, 2048),
+                                   (129, 400, 512), (200, 4096, 704), (512, 2048, 1536), (384, 6144, 512)])
+def test_linear(device, dtype, M, N, K):
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K + 8, generator=g).to(dtype).to(device)[:, :K]  # strided rows
+    w = (torch.randn(2 * N, K, generator=g) * 0.05).to(dtype).to(device)
+    ref = x.double() @ w.double().t()
+    mag = x.double().abs() @ w.double().abs().t()
+    own = mag * K * 2.0 ** -24 / 8 + 1e-9
+    half = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    y32 = ops.linear(x, w[:N], out_f32=True)
+    y = ops.linear(x, w[:N])
+    z = ops.linear(x, w, swiglu=True)
+    assert ((y32.double() - ref[:, :N]).abs() <= own[:, :N]).all()
+    assert torch.equal(y, y32.to(dtype))
+    gate, up = ref[:, :N], ref[:, N:]
+    sw = gate * torch.sigmoid(gate) * up
+    # gate and up are rounded once each, |d silu| <= 1.1 |d gate| and |silu| <= |gate|; the exponential's own
+    # error 2^-21 of the result; fp16's subnormal step
+    dg, du = own[:, :N] + half * gate.abs(), own[:, N:] + half * up.abs()
+    tol = sw.abs() * (1.01 * half + 2.0 ** -21) + 1.01 * (1.1 * dg * up.abs() + gate.abs() * du) + 2.0 ** -24
+    assert ((z.double() - sw).abs() <= tol).all()
+
+
+def test_linear_refuses(device):
+    x = torch.zeros(4, 512, device=device, dtype=torch.bfloat16)
+    w = torch.zeros(24, 512, device=device, dtype=torch.bfloat16)
+    for a, b in ((x, w), (x.float(), w[:16].float()), (x[:, :448], w[:16, :448]), (x[:, 1:], w[:16, 1:])):
+        assert not ops.linear_supported(a, b)
+        with pytest.raises(ValueError):
+            ops.linear(a, b)
+    assert ops.linear(x[:0], w[:16]).shape == (0, 16)

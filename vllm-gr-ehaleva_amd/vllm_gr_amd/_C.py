@@ -97,6 +97,7 @@ SIGNATURES = {
         _P, _I, _I,                     # slot_mapping, block_size, num_tokens
         _I, _I, _I, _F, _I, _P, _P,     # Hq, Hkv, head_dim, eps, dtype, dev_status, stream
     ]),
+    "gr_linear": (_I, [_P, _L, _P, _L, _P, _L, _I, _I, _I, _I, _I, _I, _P]),
     "gr_silu_mul": (_I, [_P, _L, _P, _L, _I, _I, _I, _P]),
     "gr_reshape_and_cache": (_I, [
         _P, _L, _P, _L, _P, _P, _L, _L, _L, _L, _P, _I, _I, _I, _I, _I, _P, _P,

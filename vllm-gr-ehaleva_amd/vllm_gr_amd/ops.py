@@ -608,6 +608,30 @@ def _rows(name: str, t: torch.Tensor) -> None:
         raise ValueError(f"{name} must be a [tokens, features] tensor with contiguous features")
 
 
+def linear_supported(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> bool:
+    """Whether ``linear`` takes these operands (see ``gr_linear`` in
+    gr_decoder.h)."""
+    n, k = w.shape
+    return (x.dtype in (torch.bfloat16, torch.float16) and w.dtype == x.dtype and x.dim() == 2 and x.shape[1] == k
+            and k % 64 == 0 and k >= 512 and n % (32 if swiglu else 16) == 0 and x.stride(1) == 1 and w.stride(1) == 1
+            and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.stride(0) >= k and w.stride(0) >= k
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and x.shape[0] <= 65536)
+
+
+def linear(x: torch.Tensor, w: torch.Tensor, *, swiglu: bool = False, out_f32: bool = False) -> torch.Tensor:
+    """``x [T, K] @ w[N, K].T`` with float32 sums; ``swiglu``: ``silu(gate) * up``
+    of the two halves of ``w``'s rows; ``out_f32``: float32 results."""
+    dev = _need_cuda(x, w)
+    if not linear_supported(x, w, swiglu):
+        raise ValueError("linear: operands outside gr_linear's range")
+    n = w.shape[0] // 2 if swiglu else w.shape[0]
+    out = torch.empty((x.shape[0], n), dtype=torch.float32 if out_f32 else x.dtype, device=dev)
+    code = _C.lib().gr_linear(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
+                              x.shape[0], n, w.shape[1], int(swiglu), int(out_f32), _dtype_code(x), _stream(dev))
+    _C.check("gr_linear", code)
+    return out
+
+
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, residual: torch.Tensor | None = None,
              out: torch.Tensor | None = None) -> torch.Tensor:
     """``out = RMSNorm(x [+ residual]) * weight``; with ``residual`` the sum is
