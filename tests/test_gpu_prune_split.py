@@ -73,3 +73,21 @@ def test_split_rows_f64_lists(device):
     torch.cuda.synchronize()
     for x, y in zip(*res):
         assert np.array_equal(_bits(x), _bits(y))
+
+
+@pytest.mark.parametrize("W,k,V", [(1, 1, 64), (32, 128, 1024), (33, 124, 1024), (200, 20, 256), (600, 6, 128)])
+@pytest.mark.parametrize("kind", ["plain", "dead", "collapse", "empty"])
+def test_one_group_merge(device, W, k, V, kind):
+    """Requests whose candidates fit one merge group (W k <= 4096): dead rows
+    (-inf scores), scores that round to one value, and too few candidates."""
+    wl = workloads.make_prune(R=3, W=W, V=V, k=k, seed=W + k)
+    eos = -1
+    if kind == "dead":
+        wl.cum[0, W // 2:] = float("-inf")
+        wl.cum[1] = float("-inf")
+    elif kind == "collapse":
+        wl.cum.fill_(-1e15)
+    elif kind == "empty":
+        eos = 5
+        wl.logits[:, :, eos] += 30.0  # with k = 1 no candidate is left
+    _check(wl, device, eos)

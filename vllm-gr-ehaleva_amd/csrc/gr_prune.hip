@@ -1235,6 +1235,11 @@ constexpr int MG_TOP_ROWS = 8;    // rows whose merged top-k bounds the group's 
 constexpr int MG_MAX_ROWS = 128;  // rows a group may hold on the bounded path
 constexpr int MG_MAX_EXTRA = 64;  // other rows' entries at or above the bound, merged one by one
 
+// DIRECT: one group holds the whole request, so its list is the result and is
+// written out as such: no second stage.  4 requests x 32 beams, k = 32: the two
+// merge launches 6.2 + 4.8 us became one of about the first's time (the
+// whole call at 151936 logits 51.0 -> 46.6 us).
+template <bool DIRECT>
 __global__ __launch_bounds__(MG_THREADS) void prune_merge_part(PruneArgs a) {
   __shared__ uint64_t mk[2][MG_GROUP_CAND];        // [0]: the group's keys by position; then merge lists
   __shared__ unsigned short mi[2][MG_GROUP_CAND];  // position in the group of each merge-list entry
@@ -1338,6 +1343,17 @@ __global__ __launch_bounds__(MG_THREADS) void prune_merge_part(PruneArgs a) {
   }
   __syncthreads();
   const int64_t o = ((int64_t)r * a.ng + g) * k;
+  // list entry `rank`: candidate (beam b, token v) with its key, or empty (key 0)
+  auto put = [&](int rank, uint64_t key, int b, int v) {
+    if constexpr (DIRECT) {
+      a.parent[o + rank] = key != 0 ? b : -1;
+      a.token[o + rank] = key != 0 ? v : -1;
+      put_score(a, o + rank, key != 0 ? dval(key) : -INFINITY);
+    } else {
+      a.part_key[o + rank] = key;
+      if (key != 0) a.part_flat[o + rank] = (int64_t)b * a.V + v;
+    }
+  };
   if (bounded && unsorted == 0) {
     // (1) the top-k of the MG_TOP_ROWS rows' union by a tournament of sorted
     // lists: each level merges lists 2j and 2j+1, keeping the first k of each
@@ -1426,10 +1442,7 @@ __global__ __launch_bounds__(MG_THREADS) void prune_merge_part(PruneArgs a) {
       // it; an extra's count of F entries before it (binary search) plus the
       // extras before it
       auto out = [&](int rank, uint64_t key, int pos) {
-        if (rank < k) {
-          a.part_key[o + rank] = key;
-          if (key != 0) a.part_flat[o + rank] = (int64_t)(b0 + div_small(pos, k1, rk1)) * a.V + mtok[pos];
-        }
+        if (rank < k) put(rank, key, b0 + div_small(pos, k1, rk1), mtok[pos]);
       };
       if (tid < fl) {
         const uint64_t ke = fk[tid];
@@ -1446,7 +1459,7 @@ __global__ __launch_bounds__(MG_THREADS) void prune_merge_part(PruneArgs a) {
         for (int j = 0; j < nx; ++j) rank += xk[j] > ke || (xk[j] == ke && xi[j] < ie);
         out(rank, ke, ie);
       }
-      for (int i = fl + nx + tid; i < k; i += MG_THREADS) a.part_key[o + i] = 0;
+      for (int i = fl + nx + tid; i < k; i += MG_THREADS) put(i, 0, 0, 0);
       return;
     }
   }
@@ -1501,10 +1514,10 @@ __global__ __launch_bounds__(MG_THREADS) void prune_merge_part(PruneArgs a) {
   __syncthreads();
   for (int i = tid; i < nsel; i += MG_THREADS) {
     const int rank = hist[i];
-    a.part_key[o + rank] = fkeys[i];
-    a.part_flat[o + rank] = ffl[i];
+    const int b = (int)(ffl[i] / a.V);
+    put(rank, fkeys[i], b, (int)(ffl[i] - (int64_t)b * a.V));
   }
-  for (int i = nsel + tid; i < a.k; i += MG_THREADS) a.part_key[o + i] = 0;
+  for (int i = nsel + tid; i < a.k; i += MG_THREADS) put(i, 0, 0, 0);
 }
 
 template <int NT, int MPT>  // threads, candidates per thread: ng * k <= MPT * NT
@@ -1803,7 +1816,11 @@ static gr_status_t prune_launch(PruneArgs& a, const float* logits, int64_t logit
     hipLaunchKernelGGL(prune_merge<0>, dim3((unsigned)num_reqs), dim3(MG_THREADS), 0, stream, a);
     return launch_status();
   }
-  hipLaunchKernelGGL(prune_merge_part, dim3((unsigned)(num_reqs * a.ng)), dim3(MG_THREADS), 0, stream, a);
+  if (a.ng == 1) {  // one group a request: its list is the result
+    hipLaunchKernelGGL(prune_merge_part<true>, dim3((unsigned)num_reqs), dim3(MG_THREADS), 0, stream, a);
+    return launch_status();
+  }
+  hipLaunchKernelGGL(prune_merge_part<false>, dim3((unsigned)(num_reqs * a.ng)), dim3(MG_THREADS), 0, stream, a);
   st = launch_status();
   if (st != GR_OK) return st;
   if (per_req <= MG_LIST_MAX)
