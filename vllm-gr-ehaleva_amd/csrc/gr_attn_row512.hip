@@ -30,9 +30,9 @@
 // tiles.
 //
 // Measured (MI355X, whole call, the generic kernel -> this one): float32, 1
-// request x 32 beams, 512-token prompt, 16 / 4 heads: 174.6 -> 21.7 us; bf16
+// request x 32 beams, 512-token prompt, 16 / 4 heads: 174 -> 21.4 us; bf16
 // head_dim 256, 4 requests x 64 beams, 1024-token prompts, 16 / 8 heads, soft
-// cap: 557 -> 25.1 us.  Error against float64: 5.7e-7 -> 4.2e-7 and 1.7e-3
+// cap: 557 -> 24.6 us (21.8 and 25.1 before the prologue's loads overlapped).  Error against float64: 5.7e-7 -> 4.2e-7 and 1.7e-3
 // (output rounding) both.
 //
 // Precision: scores, probabilities and sums are float32.  A 16-bit PV takes
@@ -158,48 +158,30 @@ __global__ __launch_bounds__(R5_THREADS) void decode_row512(DecodeArgs a, int un
   const int pre_cap = a.prefix_bt_stride * a.bs;
   const int nb0 = a.beam_start[r];
   const int W = a.beam_start[r + 1] - nb0;
+  const int P = a.prefix_len[r];
+  __asm__ volatile("" ::"s"(P));  // read with the beam range, not after its checks
   if (nb0 < 0 || W < 0 || nb0 + W > a.num_beams || W > a.max_beams) {
     if (t == 0 && chunk == 0) flag_status(a.dev_status, GR_DEV_BAD_LENGTH);
     return;
   }
   if (row0 >= W * TG) return;
   const int nrows = min(R5_ROWS, W * TG - row0);
-  const int P = a.prefix_len[r], Pc = min(max(P, 0), pre_cap);
+  const int Pc = min(max(P, 0), pre_cap);
   if (t == 0 && chunk == 0 && Pc != P) flag_status(a.dev_status, GR_DEV_BAD_LENGTH);
   const int b_lo = row0 / TG;
   const int nbm = (row0 + nrows - 1) / TG - b_lo + 1;  // beams in the chunk (<= 16)
-  if (t < nbm) {
-    const int n = nb0 + b_lo + t;
-    const int L = a.suffix_len[n], s0 = a.suffix_start ? a.suffix_start[n] : 0;
-    const int suf_cap = a.suffix_bt_stride * a.bs;
-    const int Lc = (L < 0 || s0 < 0 || s0 + L > suf_cap) ? 0 : L;
-    if (Lc != L) flag_status(a.dev_status, GR_DEV_BAD_LENGTH);
-    c_len[t] = Lc;
-    c_s0[t] = s0;
-  }
-  __syncthreads();
-  if (t == 0) {
-    int c = 0;
-    for (int j = 0; j < nbm; ++j) {
-      c_cum[j] = c;
-      c += c_len[j];
-    }
-    c_cum[nbm] = c;
-  }
-  __syncthreads();
-  const int total = Pc + c_cum[nbm];
-  const int n_tiles = (total + R5_KEYS - 1) / R5_KEYS;
-
-  const uint8_t* kc = static_cast<const uint8_t*>(a.k_cache) + (int64_t)hk * a.kv_head_stride * (int)sizeof(S);
-  const uint8_t* vc = static_cast<const uint8_t*>(a.v_cache) + (int64_t)hk * a.kv_head_stride * (int)sizeof(S);
+  // the wave's first tile's block ids where they are the prefix's, and Q, in
+  // flight under the suffix lengths' round trip
+  const int kk0 = wave * R5_KEYS + lane;
+  int blk0 = -1;
+  if (lane < R5_KEYS && kk0 < Pc)
+    blk0 = a.prefix_bt[(int64_t)r * a.prefix_bt_stride + (a.bs_shift >= 0 ? kk0 >> a.bs_shift : kk0 / a.bs)];
   const uint8_t* zero = reinterpret_cast<const uint8_t*>(g_zero16);
-
   // this lane's row and its Q: chunks 4 j + g
   const bool row_ok = m16 < nrows;
   const int rho = row0 + (row_ok ? m16 : 0);
   const int my_b = rho / TG - b_lo, my_qi = (rho / G) % a.T, my_g = rho % G;
   const int64_t my_tok = (int64_t)(nb0 + b_lo + my_b) * a.T + my_qi;
-  const int my_last = c_len[my_b] - a.T + my_qi;  // last suffix index the row sees
   u32x4_t qf[8];
   {
     const uint8_t* qp = static_cast<const uint8_t*>(a.q) +
@@ -208,12 +190,36 @@ __global__ __launch_bounds__(R5_THREADS) void decode_row512(DecodeArgs a, int un
     for (int j = 0; j < 8; ++j)
       qf[j] = *reinterpret_cast<const u32x4_t*>(row_ok ? qp + (4 * j + qd) * 16 : zero);
   }
+  // wave 0: the chunk's beams' suffix lengths and their running sum
+  if (wave == 0) {
+    int Lc = 0;
+    if (lane < nbm) {
+      const int n = nb0 + b_lo + lane;
+      const int L = a.suffix_len[n], s0 = a.suffix_start ? a.suffix_start[n] : 0;
+      const int suf_cap = a.suffix_bt_stride * a.bs;
+      Lc = (L < 0 || s0 < 0 || s0 + L > suf_cap) ? 0 : L;
+      if (Lc != L) flag_status(a.dev_status, GR_DEV_BAD_LENGTH);
+      c_len[lane] = Lc;
+      c_s0[lane] = s0;
+    }
+    const int incl = wave_incl_scan<32>(Lc);
+    if (lane < nbm) c_cum[lane + 1] = incl;
+    if (lane == 0) c_cum[0] = 0;
+  }
+  __syncthreads();
+  const int total = Pc + c_cum[nbm];
+  const int n_tiles = (total + R5_KEYS - 1) / R5_KEYS;
+
+  const uint8_t* kc = static_cast<const uint8_t*>(a.k_cache) + (int64_t)hk * a.kv_head_stride * (int)sizeof(S);
+  const uint8_t* vc = static_cast<const uint8_t*>(a.v_cache) + (int64_t)hk * a.kv_head_stride * (int)sizeof(S);
+
+  const int my_last = c_len[my_b] - a.T + my_qi;  // last suffix index the row sees
 
   // key kk of tile ti (lanes 0 .. 31 one key each): its block id, then its
   // table entries; the id's load is apart from its use so that it can be in
   // flight under other work
   struct KeyRef { int blk, o, beam, pos; };
-  auto key_ref = [&](int ti) {
+  auto key_ref = [&](int ti, bool first = false) {
     KeyRef k{-1, 0, -2, 0};
     const int kk = ti * R5_KEYS + lane;
     if (lane < R5_KEYS && kk < total) {
@@ -231,7 +237,7 @@ __global__ __launch_bounds__(R5_THREADS) void decode_row512(DecodeArgs a, int un
       }
       const int bi = a.bs_shift >= 0 ? pos >> a.bs_shift : pos / a.bs;
       k.o = pos - bi * a.bs;
-      k.blk = bt[bi];
+      k.blk = first && k.beam == -1 ? blk0 : bt[bi];
     }
     return k;
   };
@@ -265,7 +271,7 @@ __global__ __launch_bounds__(R5_THREADS) void decode_row512(DecodeArgs a, int un
   float mrow = -INFINITY, lsum = 0.f;  // the row's running maximum; this lane's keys' weights
 
   if (wave < n_tiles) {
-    key_store(0, key_ref(wave));
+    key_store(0, key_ref(wave, true));
     k_load(0);
   }
   int buf = 0;
