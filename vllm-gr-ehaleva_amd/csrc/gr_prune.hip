@@ -105,6 +105,14 @@ __device__ inline double dval(uint64_t k) {
   return __builtin_bit_cast(double, (k >> 63) ? (k & ~(1ull << 63)) : ~k);
 }
 
+// What the slices of a long row find out about it.
+struct SliceRow {
+  int32_t n;    // survivors found (may exceed PR_SURV)
+  float m;      // the row's maximum
+  uint32_t t0;  // the survivors' bound as a key
+  int32_t pad;
+};
+
 struct PruneArgs {
   const float* logits;
   int64_t row_stride;
@@ -125,13 +133,6 @@ struct PruneArgs {
   uint64_t* part_key;  // [R, ng, k] stage-1 selections: score key (0 = empty) ...
   int64_t* part_flat;  // ... and flat index b * V + v
   int ng, gr;          // row groups per request, rows per group
-  // long rows split over workgroups (prune_slice_max / prune_slice_sum), per row:
-  float* sl_max;       // [SL_MAX] maxima of disjoint parts of the row
-  float* sl_acc;       // [PR_THREADS] exp-sum partials in prune_rows' thread order
-  uint64_t* sl_surv;   // [PR_SURV] survivors: (logit bits, token)
-  int32_t* sl_n;       // survivors found (may exceed PR_SURV)
-  float* sl_m;         // the row's maximum
-  uint32_t* sl_t0;     // the survivors' bound as a key
   // catalog (nullable): the trie in CSR form -- node n's children are
   // child_token / child_node[node_start[n] .. node_start[n+1]), tokens
   // ascending; beam_node[b] is beam b's node (-1: no valid continuation)
@@ -141,7 +142,14 @@ struct PruneArgs {
   const int32_t* child_node;
   int num_nodes, num_edges;
   int32_t* dev_status;
+  // long rows split over workgroups (prune_slice_max / prune_slice_sum), per row
+  // (at the end, and few enough that the block stays four 64-byte lines):
+  float* sl_max;      // [SL_MAX] maxima of disjoint parts of the row
+  float* sl_acc;      // [PR_THREADS] exp-sum partials in prune_rows' thread order
+  uint64_t* sl_surv;  // [PR_SURV] survivors: (logit bits, token)
+  SliceRow* sl_row;
 };
+static_assert(sizeof(PruneArgs) <= 256, "four lines");
 
 // Output slot o of the selection: the float64 score, or its float32 rounding.
 __device__ inline void put_score(const PruneArgs& a, int64_t o, double v) {
@@ -439,7 +447,7 @@ __global__ __launch_bounds__(PR_THREADS) void prune_slice_max(PruneArgs a) {
     m = fmaxf(m, fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])));
   }
   a.sl_max[(int64_t)row * SL_MAX + slice * PR_THREADS + tid] = m;
-  if (slice == 0 && tid == 0) a.sl_n[row] = 0;
+  if (slice == 0 && tid == 0) a.sl_row[row].n = 0;
 }
 
 __global__ __launch_bounds__(PR_THREADS) void prune_slice_sum(PruneArgs a) {
@@ -523,8 +531,8 @@ __global__ __launch_bounds__(PR_THREADS) void prune_slice_sum(PruneArgs a) {
   if (t0 <= fkey(-INFINITY)) t0 = 0;
   const float t0f = t0 == 0 ? -INFINITY : fval(t0);
   if (slice == 0 && tid == 0) {
-    a.sl_m[row] = m;
-    a.sl_t0[row] = t0;
+    a.sl_row[row].m = m;
+    a.sl_row[row].t0 = t0;
   }
 
   const float ml = m * 0x1.715476p+0f;
@@ -574,7 +582,7 @@ __global__ __launch_bounds__(PR_THREADS) void prune_slice_sum(PruneArgs a) {
       const int n = list.n;
       int base = 0;
       // (a list that overflowed sends the row to the radix path, whatever the other slices hold)
-      if (lane == 0 && n > 0) base = atomicAdd(&a.sl_n[row], n <= SL_LIST ? n : PR_SURV + 1);
+      if (lane == 0 && n > 0) base = atomicAdd(&a.sl_row[row].n, n <= SL_LIST ? n : PR_SURV + 1);
       base = __builtin_amdgcn_readfirstlane(base);
       for (int i = lane; i < min(n, SL_LIST); i += 64)
         if (base + i < PR_SURV) a.sl_surv[(int64_t)row * PR_SURV + base + i] = list.raw[i];
@@ -654,7 +662,7 @@ __global__ __launch_bounds__(PR_THREADS) void prune_rows(PruneArgs a) {
   // other than the thread maximum: it tightens the selection bound below) ----
   float tm = -INFINITY, t2 = -INFINITY, m;
   if constexpr (SPLIT) {
-    m = a.sl_m[row];
+    m = a.sl_row[row].m;
   } else {
     PR_FOR_CHUNKS(c) {
       if (live(c)) {
@@ -714,7 +722,7 @@ __global__ __launch_bounds__(PR_THREADS) void prune_rows(PruneArgs a) {
   // directly.
   uint32_t t0 = 0;
   if constexpr (SPLIT) {
-    t0 = a.sl_t0[row];
+    t0 = a.sl_row[row].t0;
   } else if (k1 <= PR_THREADS) {
     const int kw = (k1 + 3) >> 2;
     const uint32_t a0 = fkey(tm) >> 16;  // the top 16 bits of the key suffice for a bound
@@ -746,7 +754,7 @@ __global__ __launch_bounds__(PR_THREADS) void prune_rows(PruneArgs a) {
   }
   int n_surv;
   if constexpr (SPLIT) {
-    n_surv = __builtin_amdgcn_readfirstlane(a.sl_n[row]);
+    n_surv = __builtin_amdgcn_readfirstlane(a.sl_row[row].n);
     if (n_surv <= PR_SURV)
       for (int i = tid; i < n_surv; i += PR_THREADS) sk[i] = a.sl_surv[(int64_t)row * PR_SURV + i];
   } else {
@@ -1350,8 +1358,7 @@ __global__ __launch_bounds__(MG_THREADS) void prune_merge_part(PruneArgs a) {
       a.token[o + rank] = key != 0 ? v : -1;
       put_score(a, o + rank, key != 0 ? dval(key) : -INFINITY);
     } else {
-      a.part_key[o + rank] = key;
-      if (key != 0) a.part_flat[o + rank] = (int64_t)b * a.V + v;
+      a.part_key[o + rank] = key;  // (only empty entries come here)
     }
   };
   if (bounded && unsorted == 0) {
@@ -1442,7 +1449,14 @@ __global__ __launch_bounds__(MG_THREADS) void prune_merge_part(PruneArgs a) {
       // it; an extra's count of F entries before it (binary search) plus the
       // extras before it
       auto out = [&](int rank, uint64_t key, int pos) {
-        if (rank < k) put(rank, key, b0 + div_small(pos, k1, rk1), mtok[pos]);
+        if (rank < k) {
+          if constexpr (DIRECT) {
+            put(rank, key, b0 + div_small(pos, k1, rk1), mtok[pos]);
+          } else {
+            a.part_key[o + rank] = key;
+            if (key != 0) a.part_flat[o + rank] = (int64_t)(b0 + div_small(pos, k1, rk1)) * a.V + mtok[pos];
+          }
+        }
       };
       if (tid < fl) {
         const uint64_t ke = fk[tid];
@@ -1514,8 +1528,13 @@ __global__ __launch_bounds__(MG_THREADS) void prune_merge_part(PruneArgs a) {
   __syncthreads();
   for (int i = tid; i < nsel; i += MG_THREADS) {
     const int rank = hist[i];
-    const int b = (int)(ffl[i] / a.V);
-    put(rank, fkeys[i], b, (int)(ffl[i] - (int64_t)b * a.V));
+    if constexpr (DIRECT) {
+      const int b = (int)(ffl[i] / a.V);
+      put(rank, fkeys[i], b, (int)(ffl[i] - (int64_t)b * a.V));
+    } else {
+      a.part_key[o + rank] = fkeys[i];
+      a.part_flat[o + rank] = ffl[i];
+    }
   }
   for (int i = nsel + tid; i < a.k; i += MG_THREADS) put(i, 0, 0, 0);
 }
@@ -1713,7 +1732,7 @@ static bool split_rows(size_t rows, int vocab, int k) {
 }
 static size_t split_bytes(size_t rows) {
   return align256(rows * SL_MAX * sizeof(float)) + align256(rows * PR_THREADS * sizeof(float)) +
-         align256(rows * PR_SURV * sizeof(uint64_t)) + 3 * align256(rows * sizeof(int32_t));
+         align256(rows * PR_SURV * sizeof(uint64_t)) + align256(rows * sizeof(SliceRow));
 }
 
 extern "C" size_t gr_beam_prune_workspace_size_split(int num_reqs, int beam_width, int vocab, int k) {
@@ -1789,11 +1808,7 @@ static gr_status_t prune_launch(PruneArgs& a, const float* logits, int64_t logit
     p += align256(rows * PR_THREADS * sizeof(float));
     a.sl_surv = reinterpret_cast<uint64_t*>(p);
     p += align256(rows * PR_SURV * sizeof(uint64_t));
-    a.sl_n = reinterpret_cast<int32_t*>(p);
-    p += align256(rows * sizeof(int32_t));
-    a.sl_m = reinterpret_cast<float*>(p);
-    p += align256(rows * sizeof(float));
-    a.sl_t0 = reinterpret_cast<uint32_t*>(p);
+    a.sl_row = reinterpret_cast<SliceRow*>(p);
     hipLaunchKernelGGL(prune_slice_max, dim3((unsigned)(rows * SL_NS)), dim3(PR_THREADS), 0, stream, a);
     hipLaunchKernelGGL(prune_slice_sum, dim3((unsigned)(rows * SL_NS)), dim3(PR_THREADS), 0, stream, a);
     if (cat) hipLaunchKernelGGL((prune_rows<0, true, false, true>), dim3((unsigned)rows), dim3(PR_THREADS), 0, stream, a);
