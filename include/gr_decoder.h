@@ -55,10 +55,11 @@ gr_status_t gr_qk_norm_rope_cache(
 /*
  * Projection: out[t, n] = round(sum_k x[t, k] w[n, k]) for x [num_tokens,
  * in_features] and w [out_features, in_features] (nn.Linear's layout, no bias),
- * bf16 or fp16 with float32 sums; out in the inputs' type, or float32 with
- * out_f32.  swiglu: w is [2 * out_features, in_features] (gate | up) and out[t,
- * n] = round(silu(gate) * up) of the sums rounded to the inputs' type.  Made for the few hundred rows of a
- * decode step; needs 16-byte aligned rows, in_features % 64 == 0 and >= 512,
+ * bf16 or fp16 with float32 sums; out in the inputs' type, float32 (out_f32 =
+ * 1), or float32 holding the values that the inputs' type would (out_f32 = 2).
+ * swiglu: w is [2 * out_features, in_features] (gate | up) and out[t, n] =
+ * round(silu(gate) * up) of the sums rounded to the inputs' type.  Made for the
+ * few hundred rows of a decode step; needs 16-byte aligned rows, in_features % 64 == 0 and >= 512,
  * out_features % 16 == 0 (GR_ERR_UNSUPPORTED otherwise, and for float32).
  */
 gr_status_t gr_linear(void* out, int64_t out_stride, const void* x, int64_t x_stride, const void* w,

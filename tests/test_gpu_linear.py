@@ -11,6 +11,7 @@ import pytest
 import torch
 
 from vllm_gr_amd import ops
+from vllm_gr_amd.v1.sid_decoder import DecoderConfig, SidDecoder, init_weights
 
 pytestmark = pytest.mark.gpu
 
@@ -48,3 +49,25 @@ def test_linear_refuses(device):
         with pytest.raises(ValueError):
             ops.linear(a, b)
     assert ops.linear(x[:0], w[:16]).shape == (0, 16)
+
+
+def _decoder(device, dtype=torch.bfloat16, vocab=208):
+    cfg = DecoderConfig(num_layers=1, hidden=512, num_heads=4, num_kv_heads=2, ffn=512, vocab=vocab, dtype=dtype)
+    return SidDecoder(cfg, init_weights(cfg, 3, device), max_position=8)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_logits_are_rounded_alike_at_every_row_count(device, dtype):
+    """Logits are the model type's values in float32, on either side of the row
+    count from which the library computes them: a beam's score, and a tie of two
+    of them, is not a matter of how many requests share the step."""
+    dec = _decoder(device, dtype)
+    hidden = torch.randn(513, 512, generator=torch.Generator().manual_seed(2)).to(dtype).to(device)
+    want = (hidden.double() @ dec.w["lm_head"].double().t())
+    mag = hidden.double().abs() @ dec.w["lm_head"].double().abs().t()
+    half = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for rows in (1, 8, 200, 512, 513):
+        got = dec.compute_logits(hidden[:rows])
+        assert got.dtype == torch.float32 and torch.equal(got, got.to(dtype).float()), rows
+        tol = want[:rows].abs() * half * 1.01 + mag[:rows] * 512 * 2.0 ** -24 / 8 + 2.0 ** -25
+        assert ((got.double() - want[:rows]).abs() <= tol).all(), rows

@@ -51,7 +51,7 @@ struct LinearArgs {
   int64_t w_stride;
   int M, N, K;  // N: output columns (the weights have 2 N rows with SWIGLU: gate, then up)
   int tiles_m, tiles_n;
-  int out_f32;
+  int out_f32;  // 0: the inputs' type; 1: float32; 2: float32 of the inputs' type
 };
 
 template <int DT> __device__ inline lf4_t mma32(u32x4_t a, u32x4_t b, lf4_t c) {
@@ -195,8 +195,12 @@ __global__ __launch_bounds__(LN_THREADS, 1) void linear_k(LinearArgs a) {
   auto put = [&](int t, int col, const float (&v)[4]) {
     if (t >= a.M || col >= a.N) return;
     if (a.out_f32) {
-      *reinterpret_cast<lf4_t*>(static_cast<float*>(a.out) + (int64_t)t * a.out_stride + col) =
-          lf4_t{v[0], v[1], v[2], v[3]};
+      lf4_t f = {v[0], v[1], v[2], v[3]};
+      if (a.out_f32 == 2) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) f[u] = Elem<DT>::to_float(Elem<DT>::from_float(f[u]));
+      }
+      *reinterpret_cast<lf4_t*>(static_cast<float*>(a.out) + (int64_t)t * a.out_stride + col) = f;
     } else {
       *reinterpret_cast<u32x2_t*>(static_cast<S*>(a.out) + (int64_t)t * a.out_stride + col) =
           u32x2_t{Mma<DT>::pack2(v[0], v[1]), Mma<DT>::pack2(v[2], v[3])};
@@ -281,7 +285,7 @@ extern "C" gr_status_t gr_linear(void* out, int64_t out_stride, const void* x, i
                                  int64_t w_stride, int num_tokens, int out_features, int in_features, int swiglu,
                                  int out_f32, int dtype, hipStream_t stream) {
   if (num_tokens < 0 || out_features < 1 || in_features < 1 || (swiglu != 0 && swiglu != 1) ||
-      (out_f32 != 0 && out_f32 != 1) || !dtype_valid(dtype))
+      out_f32 < 0 || out_f32 > 2 || !dtype_valid(dtype))
     return GR_ERR_INVALID_ARG;
   if (num_tokens == 0) return GR_OK;
   if (!out || !x || !w || out_stride < out_features || x_stride < in_features || w_stride < in_features)

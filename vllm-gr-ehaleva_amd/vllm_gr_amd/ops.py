@@ -618,16 +618,19 @@ def linear_supported(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> 
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and x.shape[0] <= 65536)
 
 
-def linear(x: torch.Tensor, w: torch.Tensor, *, swiglu: bool = False, out_f32: bool = False) -> torch.Tensor:
+def linear(x: torch.Tensor, w: torch.Tensor, *, swiglu: bool = False, out_f32: bool = False,
+           rounded: bool = False) -> torch.Tensor:
     """``x [T, K] @ w[N, K].T`` with float32 sums; ``swiglu``: ``silu(gate) * up``
-    of the two halves of ``w``'s rows; ``out_f32``: float32 results."""
+    of the two halves of ``w``'s rows; ``out_f32``: float32 results, with
+    ``rounded`` the values that ``x``'s type would hold."""
     dev = _need_cuda(x, w)
     if not linear_supported(x, w, swiglu):
         raise ValueError("linear: operands outside gr_linear's range")
     n = w.shape[0] // 2 if swiglu else w.shape[0]
     out = torch.empty((x.shape[0], n), dtype=torch.float32 if out_f32 else x.dtype, device=dev)
     code = _C.lib().gr_linear(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
-                              x.shape[0], n, w.shape[1], int(swiglu), int(out_f32), _dtype_code(x), _stream(dev))
+                              x.shape[0], n, w.shape[1], int(swiglu), (2 if rounded else 1) if out_f32 else 0, _dtype_code(x),
+                              _stream(dev))
     _C.check("gr_linear", code)
     return out
 

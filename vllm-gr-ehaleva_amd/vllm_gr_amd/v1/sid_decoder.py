@@ -12,7 +12,7 @@ from N(0, std) -- there are no checkpoints here:
   the caller gives, attention through the BeamAttention backend, o
   projection, residual add; RMSNorm, SwiGLU MLP (silu(gate) * up, down),
   residual add;
-* final RMSNorm; logits = lm_head rows in float32.
+* final RMSNorm; logits = lm_head products in ``cfg.dtype``, widened to float32.
 
 The projections of up to 512 rows from at most 2048 features -- a decode
 step's qkv, o, gate_up (with its SiLU gate) and lm_head -- are gr_linear; the
@@ -188,5 +188,9 @@ class SidDecoder:
         return ops.rms_norm(mlp, w["final_norm"], eps, residual=h)
 
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
+        # the model type's values on either path: scores and their ties do not
+        # depend on how many rows share the step
         w = self.w["lm_head"]
-        return ops.linear(hidden, w, out_f32=True) if _own_linear(hidden, w) else F.linear(hidden, w).float()
+        if _own_linear(hidden, w):
+            return ops.linear(hidden, w, out_f32=True, rounded=True)
+        return F.linear(hidden, w).float()
