@@ -97,3 +97,51 @@ def test_row512_infinite_value_row(device, dtype, D):
     wl.kv_cache[1, blk, 3, 1] = -float("inf")
     out, _ = _run(wl, device)
     assert (out[:, 0] == np.inf).all() and (out[:, 1] == -np.inf).all()
+
+
+@pytest.mark.parametrize("dtype,D", DTYPES)
+def test_row512_weights_keep_float32(device, dtype, D):
+    """Two keys of nearly equal weight whose V rows cancel: the result is the
+    difference of the weights, which terms of fewer bits than float32's show.
+
+    Bound: the output's rounding, plus 2^-20 (of |v| = 1) for the float32 steps
+    -- scores of at most 2 in size, rounded at 2^-23, and an exponential and sums
+    of a few float32 units."""
+    g = torch.Generator().manual_seed(D)
+    wl = workloads.make_decode(R=1, W=64, P=2, L=0, Hq=16, Hkv=2, D=D, dtype=dtype, input_scale=0.5, seed=4)
+    b = int(wl.prefix_bt[0, 0])
+    wl.kv_cache[0, b, 1] = wl.kv_cache[0, b, 0]
+    wl.kv_cache[0, b, 1, :, :4] += 0.05 * torch.randn(2, 4, generator=g).to(dtype)
+    wl.kv_cache[1, b, 0] = 1.0
+    wl.kv_cache[1, b, 1] = -1.0
+    out, _ = _run(wl, device)
+    q, k = wl.q.double().view(64, 2, 8, D), wl.kv_cache[0, b, :2].double()
+    ref = torch.tanh(torch.einsum("whgd,hd->whg", q, (k[0] - k[1])) * wl.scale / 2).reshape(64, 16, 1).numpy()
+    assert (np.abs(out - ref) <= 1.01 * HALF_ULP[dtype] * np.abs(ref) + 2.0 ** -20).all(), np.abs(out - ref).max()
+
+
+@pytest.mark.parametrize("dtype,D", DTYPES)
+def test_row512_small_weight_of_a_large_value(device, dtype, D):
+    """A weight near 2^-29 on a large V row beside a V row of zeros: the result
+    is that weight.
+
+    Bound: the output's rounding (half of fp16's subnormal step at least), plus
+    the score's error as a share of the result: a float32 sum of D products of one
+    sign, each addition rounded at 2^-24 of a running sum that is half of the whole
+    on average, and 2^-20 for the exponential and the quotient."""
+    wl = workloads.make_decode(R=1, W=16, P=2, L=0, Hq=8, Hkv=1, D=D, dtype=dtype, input_scale=1.0, seed=6)
+    b = int(wl.prefix_bt[0, 0])
+    sign = torch.randn(D, generator=torch.Generator().manual_seed(7)).sign()
+    amp = 18.0 / D ** 0.5 * (1.0 + torch.arange(128).view(16, 8, 1) / 1024.0)
+    wl.q.copy_((amp * sign).to(dtype))
+    wl.kv_cache[0, b, 0, 0] = sign.to(dtype)
+    wl.kv_cache[0, b, 1, 0] = 0.0
+    wl.kv_cache[1, b, 0, 0] = 0.0
+    wl.kv_cache[1, b, 1, 0] = 60000.0
+    out, _ = _run(wl, device)
+    s = (wl.q.double() * sign.double()).sum(-1, keepdim=True) * wl.scale
+    v = wl.kv_cache[1, b, 1, 0, 0].double()
+    ref = (v / (1.0 + torch.exp(s))).numpy()
+    sub = 2.0 ** -25 if dtype == torch.float16 else 0.0
+    own = D * 2.0 ** -24 * s.numpy() / 2 + 2.0 ** -20
+    assert (np.abs(out - ref) <= (1.01 * HALF_ULP[dtype] + own) * np.abs(ref) + sub).all(), (np.abs(out - ref) / ref).max()

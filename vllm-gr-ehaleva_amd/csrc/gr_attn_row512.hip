@@ -32,11 +32,14 @@
 // Measured (MI355X, whole call, the generic kernel -> this one): float32, 1
 // request x 32 beams, 512-token prompt, 16 / 4 heads: 174 -> 21.4 us; bf16
 // head_dim 256, 4 requests x 64 beams, 1024-token prompts, 16 / 8 heads, soft
-// cap: 557 -> 24.6 us (21.8 and 25.1 before the prologue's loads overlapped).  Error against float64: 5.7e-7 -> 4.2e-7 and 1.7e-3
-// (output rounding) both.
+// cap: 557 -> 26.2 us (24.7 with two terms a weight); fp16, the same without the
+// cap: 551 -> 28.6 us (43.4 where every tile takes the float32 MFMA).  Error
+// against float64: 5.7e-7 -> 4.2e-7 and 1.7e-3 (output rounding) both.
 //
-// Precision: scores, probabilities and sums are float32.  A 16-bit PV takes
-// each probability as two 16-bit terms (hi + lo, 16 bits of it), two MFMAs.
+// Precision: scores, probabilities and sums are float32, and PV takes all 24
+// bits of a probability: as three 16-bit terms (three MFMAs), and in fp16, whose
+// range they would leave, a tile with a probability below 2^-12 of the largest
+// through the float32 MFMA.
 #include "gr_mfma_tile.h"
 
 namespace gr {
@@ -54,13 +57,15 @@ typedef float f4_t __attribute__((__vector_size__(16)));
 template <int DT> struct Row512;
 template <> struct Row512<GR_DTYPE_F32> {
   static constexpr int PER = 4;  // elements per 16-byte chunk
-  static constexpr float PSCALE = 1.f;
+  static constexpr float PSCALE = 1.f;  // PV takes its weights times this
   __device__ static inline f4_t qk(u32x4_t k, u32x4_t q, f4_t s) {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       s = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(k[e]), __uint_as_float(q[e]), s, 0, 0, 0);
     return s;
   }
+  // element e of a V chunk
+  __device__ static inline float v_elem(u32x4_t v, int e) { return __uint_as_float(v[e]); }
   __device__ static inline u32x4_t pack(const float (&v)[4]) {
     return u32x4_t{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
   }
@@ -68,18 +73,13 @@ template <> struct Row512<GR_DTYPE_F32> {
 template <> struct Row512<GR_DTYPE_BF16> {
   static constexpr int PER = 8;
   static constexpr float PSCALE = 1.f;
+  static constexpr uint32_t HEAD = 0xffff0000u;  // sign, exponent and the leading 8 bits of a float32
+  static constexpr float TERM_MIN = 0x1p-126f;   // the smallest normal value of a term
   __device__ static inline f4_t mma(u32x4_t a, u32x4_t b, f4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
                                                    0, 0, 0);
   }
   __device__ static inline f4_t qk(u32x4_t k, u32x4_t q, f4_t s) { return mma(k, q, s); }
-  // p = hi + lo with both terms positive for p > 0, so that an infinite V row
-  // gives the infinity that a float32 weight gives it: hi is cut off (not
-  // rounded) from just below p, lo is at least 2^-9 p
-  __device__ static inline void split(float p, float& hi, float& lo) {
-    hi = __uint_as_float(__float_as_uint(p * 0x1.ffp-1f) & 0xffff0000u);
-    lo = p - hi;
-  }
   __device__ static inline u32x4_t pack(const float (&v)[8]) {
     return u32x4_t{Mma<GR_DTYPE_BF16>::pack2(v[0], v[1]), Mma<GR_DTYPE_BF16>::pack2(v[2], v[3]),
                    Mma<GR_DTYPE_BF16>::pack2(v[4], v[5]), Mma<GR_DTYPE_BF16>::pack2(v[6], v[7])};
@@ -87,25 +87,40 @@ template <> struct Row512<GR_DTYPE_BF16> {
 };
 template <> struct Row512<GR_DTYPE_F16> {
   static constexpr int PER = 8;
-  // weights are carried as 256 p (at most 256): the low terms stay normal
-  static constexpr float PSCALE = 256.f;
+  static constexpr float PSCALE = 0x1p15f;       // the largest weight near the top of fp16's range
+  static constexpr uint32_t HEAD = 0xffffe000u;  // ... and the leading 11 bits
+  static constexpr float TERM_MIN = 0x1p-24f;    // fp16's smallest value
+  // Scaled weights from 8 are sums of three terms: their last bit is 2^-20 or
+  // more, and a term raised to TERM_MIN adds 2^-27 of them at most.
+  static constexpr float SPLIT_MIN = 8.f;
   __device__ static inline f4_t mma(u32x4_t a, u32x4_t b, f4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0,
                                                   0, 0);
   }
   __device__ static inline f4_t qk(u32x4_t k, u32x4_t q, f4_t s) { return mma(k, q, s); }
-  // as for bf16; a term below fp16's range stays at its smallest value
-  // (2^-32 of the row's largest weight)
-  __device__ static inline void split(float p, float& hi, float& lo) {
-    hi = (float)(_Float16)(p * 0x1.ffp-1f);
-    hi = p > 0.f ? fmaxf(hi, 0x1p-24f) : hi;
-    lo = p > 0.f ? fmaxf(p - hi, 0x1p-24f) : p - hi;
+  __device__ static inline float v_elem(u32x4_t v, int e) {
+    return Elem<GR_DTYPE_F16>::to_float((uint16_t)(v[e >> 1] >> (16 * (e & 1))));
   }
   __device__ static inline u32x4_t pack(const float (&v)[8]) {
     return u32x4_t{Mma<GR_DTYPE_F16>::pack2(v[0], v[1]), Mma<GR_DTYPE_F16>::pack2(v[2], v[3]),
                    Mma<GR_DTYPE_F16>::pack2(v[4], v[5]), Mma<GR_DTYPE_F16>::pack2(v[6], v[7])};
   }
 };
+
+// A weight as three terms of the type, each the leading bits of what is left:
+// all 24 bits of it.  A term that would be zero beside p > 0 is raised to
+// TERM_MIN, so that an infinite V row gives the infinity that a float32 weight
+// gives it, not 0 * infinity.
+template <int DT> __device__ inline void split_weight(float p, float (&t)[3]) {
+  using M = Row512<DT>;
+  const float lo = p > 0.f ? M::TERM_MIN : 0.f;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const float h = __uint_as_float(__float_as_uint(p) & M::HEAD);
+    t[i] = fmaxf(h, lo);
+    p -= h;
+  }
+}
 
 // The row's partial outputs of one wave in LDS: 16 rows of PER * 32 floats, 16
 // bytes of padding a row (rows start on different banks).
@@ -336,37 +351,59 @@ __global__ __launch_bounds__(R5_THREADS) void decode_row512(DecodeArgs a, int un
     }
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
-      p[s] = p[s] == -INFINITY ? 0.f : expf(p[s] - mrow) * M::PSCALE;
+      p[s] = p[s] == -INFINITY ? 0.f : expf(p[s] - mrow);
       lsum += p[s];
     }
-    if constexpr (DT == GR_DTYPE_F32) {
+    if constexpr (M::PSCALE != 1.f) {
 #pragma unroll
-      for (int s = 0; s < 8; ++s)
+      for (int s = 0; s < 8; ++s) p[s] *= M::PSCALE;
+    }
+    bool terms = DT != GR_DTYPE_F32;  // 16-bit MFMAs on three terms of the weights (wave-uniform)
+    if constexpr (DT == GR_DTYPE_F16) {
+      bool small = false;
+#pragma unroll
+      for (int s = 0; s < 8; ++s) small |= (p[s] > 0.f) & (p[s] < M::SPLIT_MIN);
+      terms = __ballot(small) == 0;
+    }
+    if constexpr (DT != GR_DTYPE_F32) {
+      if (terms) {
+        float pt[3][8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+          float t[3];
+          split_weight<DT>(p[s], t);
+#pragma unroll
+          for (int i = 0; i < 3; ++i) pt[i][s] = t[i];
+        }
+        const u32x4_t pp[3] = {M::pack(pt[0]), M::pack(pt[1]), M::pack(pt[2])};
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
-          for (int e = 0; e < PER; ++e)
-            o[c][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(vf[c][s][e]), p[s], o[c][e], 0, 0, 0);
-    } else {
-      float hi[8], lo[8];
+          for (int w = 0; w < 4; ++w) {  // dims 2 w, 2 w + 1 of the chunk over the 8 keys
+            u32x4_t v0, v1;
 #pragma unroll
-      for (int s = 0; s < 8; ++s) M::split(p[s], hi[s], lo[s]);
-      const u32x4_t ph = M::pack(hi), pl = M::pack(lo);
+            for (int h = 0; h < 4; ++h) {
+              v0[h] = __builtin_amdgcn_perm(vf[c][2 * h + 1][w], vf[c][2 * h][w], 0x05040100u);
+              v1[h] = __builtin_amdgcn_perm(vf[c][2 * h + 1][w], vf[c][2 * h][w], 0x07060302u);
+            }
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {  // dims 2 w, 2 w + 1 of the chunk over the 8 keys
-          u32x4_t v0, v1;
-#pragma unroll
-          for (int h = 0; h < 4; ++h) {
-            v0[h] = __builtin_amdgcn_perm(vf[c][2 * h + 1][w], vf[c][2 * h][w], 0x05040100u);
-            v1[h] = __builtin_amdgcn_perm(vf[c][2 * h + 1][w], vf[c][2 * h][w], 0x07060302u);
+            for (int i = 2; i >= 0; --i) {  // the small terms first
+              o[c][2 * w] = M::mma(v0, pp[i], o[c][2 * w]);
+              o[c][2 * w + 1] = M::mma(v1, pp[i], o[c][2 * w + 1]);
+            }
           }
-          o[c][2 * w] = M::mma(v0, ph, o[c][2 * w]);
-          o[c][2 * w + 1] = M::mma(v1, ph, o[c][2 * w + 1]);
-          o[c][2 * w] = M::mma(v0, pl, o[c][2 * w]);
-          o[c][2 * w + 1] = M::mma(v1, pl, o[c][2 * w + 1]);
-        }
+      }
+    }
+    if constexpr (DT != GR_DTYPE_BF16) {
+      if (!terms) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int e = 0; e < PER; ++e)
+              o[c][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(M::v_elem(vf[c][s], e), p[s], o[c][e], 0, 0, 0);
+      }
     }
   }
 
@@ -406,8 +443,12 @@ __global__ __launch_bounds__(R5_THREADS) void decode_row512(DecodeArgs a, int un
   static_assert(R5_ROWS * 32 == R5_THREADS, "a thread per output chunk");
   if (orow >= nrows) return;
   const int orho = row0 + orow;
-  const int og = orho % G;
-  const int64_t otok = (int64_t)(nb0 + orho / TG) * a.T + (orho / G) % a.T;
+  // (fp16, whose loop fills the registers: opaque copies, so that the prologue's
+  // reciprocals are not spilled across the loop for these quotients)
+  int oG = G, oT = a.T;
+  if constexpr (DT == GR_DTYPE_F16) __asm__ volatile("" : "+s"(oG), "+s"(oT));
+  const int og = orho % oG;
+  const int64_t otok = (int64_t)(nb0 + orho / (oT * oG)) * oT + (orho / oG) % oT;
   const float sink = a.sinks ? a.sinks[hk * G + og] : -INFINITY;
   const float m = row_max(orow, sink);
   float l = 0.f;
@@ -416,7 +457,6 @@ __global__ __launch_bounds__(R5_THREADS) void decode_row512(DecodeArgs a, int un
     const float mw = w_m[w][orow];
     if (mw != -INFINITY) l += w_l[w][orow] * expf(mw - m);
   }
-  l *= 1.f / M::PSCALE;
   if (sink != -INFINITY) l += expf(sink - m);
   float v[PER];
 #pragma unroll
