@@ -71,3 +71,39 @@ def test_logits_are_rounded_alike_at_every_row_count(device, dtype):
         assert got.dtype == torch.float32 and torch.equal(got, got.to(dtype).float()), rows
         tol = want[:rows].abs() * half * 1.01 + mag[:rows] * 512 * 2.0 ** -24 / 8 + 2.0 ** -25
         assert ((got.double() - want[:rows]).abs() <= tol).all(), rows
+
+
+def test_logits_under_autograd_and_transforms(device):
+    """compute_logits is differentiable in the hidden states and the weights, and
+    works under vmap, forward mode and tracing, as the torch product it stands for."""
+    import torch.autograd.forward_ad as fw
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+    dec = _decoder(device)
+    w = dec.w["lm_head"]
+    h = torch.randn(6, 512, device=device, dtype=torch.bfloat16)
+    plain = lambda x, w=w: torch.nn.functional.linear(x, w).float()
+    up = torch.randn(6, 208, device=device)
+    for hg, wg in ((True, False), (False, True), (True, True)):
+        x, lm = h.clone().requires_grad_(hg), w.clone().requires_grad_(wg)
+        x2, lm2 = h.clone().requires_grad_(hg), w.clone().requires_grad_(wg)
+        dec.w["lm_head"] = lm
+        (dec.compute_logits(x) * up).sum().backward()
+        (plain(x2, lm2) * up).sum().backward()
+        for a, b in ((x, x2), (lm, lm2)):
+            assert (a.grad is None) == (b.grad is None)
+            assert a.grad is None or torch.equal(a.grad, b.grad)
+    dec.w["lm_head"] = w
+    assert torch.equal(torch.func.vmap(dec.compute_logits)(h.view(2, 3, 512)), torch.func.vmap(plain)(h.view(2, 3, 512)))
+    t = torch.randn_like(h)
+    for a, b in zip(torch.func.jvp(dec.compute_logits, (h,), (t,)), torch.func.jvp(plain, (h,), (t,))):
+        assert torch.equal(a, b)
+    with fw.dual_level():
+        assert torch.equal(fw.unpack_dual(dec.compute_logits(fw.make_dual(h, t))).tangent,
+                           fw.unpack_dual(plain(fw.make_dual(h, t))).tangent)
+    traced = make_fx(lambda x: dec.compute_logits(x))(h)
+    assert torch.equal(traced(2 * h), plain(2 * h))  # not h's logits as a constant
+    with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+        assert dec.compute_logits(mode.from_tensor(h)).shape == (6, 208)
+    with torch.no_grad():  # the usual call
+        assert not dec.compute_logits(h.clone().requires_grad_()).requires_grad

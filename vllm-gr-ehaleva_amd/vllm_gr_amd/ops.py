@@ -613,9 +613,10 @@ def linear_supported(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> 
     gr_decoder.h)."""
     n, k = w.shape
     return (x.is_cuda and w.device == x.device and x.dtype in (torch.bfloat16, torch.float16) and w.dtype == x.dtype
-            and x.dim() == 2 and x.shape[1] == k and n > 0 and k % 64 == 0 and k >= 512 and n % (32 if swiglu else 16) == 0 and x.stride(1) == 1 and w.stride(1) == 1
-            and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.stride(0) >= k and w.stride(0) >= k
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and x.shape[0] <= 65536)
+            and x.dim() == 2 and x.shape[1] == k and x.shape[0] <= 65536 and k % 64 == 0 and k >= 512
+            and n > 0 and n % (32 if swiglu else 16) == 0
+            and x.stride(1) == 1 and x.stride(0) >= k and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
+            and w.stride(1) == 1 and w.stride(0) >= k and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, *, swiglu: bool = False, out_f32: bool = False,

@@ -119,6 +119,20 @@ class RotaryEmbedding:
         self.max_pos = max_pos
 
 
+def _plain(*ts: torch.Tensor) -> bool:
+    """Whether a kernel on the tensors' addresses can stand in for a torch
+    operation: ordinary tensors, and nothing that follows torch operations --
+    an autograd graph, forward mode, vmap and the other function transforms, a
+    dispatch mode (fake tensors, tracing) or a compiler -- would miss it.  (The
+    layers of ``forward`` run such kernels throughout; ``compute_logits`` is one
+    product and keeps what the torch product does.)"""
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in ts)
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
+            and torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._len_torch_dispatch_stack() == 0
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+
+
 def _own_linear(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> bool:
     """Whether gr_linear takes a projection.  Its gains are at decode-step row
     counts and shallow depths: at 768 rows SwiGLU (2048 in, 6144 out) takes 55
@@ -191,6 +205,6 @@ class SidDecoder:
         # the model type's values on either path: scores and their ties do not
         # depend on how many rows share the step
         w = self.w["lm_head"]
-        if _own_linear(hidden, w):
+        if _plain(hidden, w) and _own_linear(hidden, w):
             return ops.linear(hidden, w, out_f32=True, rounded=True)
         return F.linear(hidden, w).float()
