@@ -67,6 +67,12 @@ gr_status_t gr_linear(void* out, int64_t out_stride, const void* x, int64_t x_st
                       int out_f32, int dtype, hipStream_t stream);
 
 /*
+ * The workgroup tile that gr_linear takes for these sizes: 1000 * rows +
+ * weight rows; 0 for sizes that are not positive.
+ */
+int gr_linear_tile(int num_tokens, int out_features, int in_features, int swiglu);
+
+/*
  * SwiGLU gate: out[t, i] = round(silu(x[t, i]) * x[t, ffn + i]) for
  * x [num_tokens, 2 * ffn] (gate | up), silu(g) = g / (1 + exp(-g)).
  * num_tokens <= 65535.

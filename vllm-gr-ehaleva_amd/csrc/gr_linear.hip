@@ -233,22 +233,27 @@ __global__ __launch_bounds__(LN_THREADS, 1) void linear_k(LinearArgs a) {
   }
 }
 
-// The tile with the least estimated time: rounds of 256 workgroups, each a
-// fixed part and its stages.  Clocks per stage from one-round launches of 32
-// and 96 stages (64 x 64: 7.0 and 21.4 us, 128 x 64: 9.7 and 28.5, 128 x 128:
-// 15.0 and 41, 128 x 192: 20.5 and 57): 25 to 35 bytes per clock into the CU,
-// which the MFMAs wait for in every tile.
-struct LinearTile { int bm, bn, clk; };
-constexpr LinearTile kLinearTiles[] = {{64, 64, 300}, {128, 64, 450}, {128, 128, 650}, {128, 192, 900}};
-constexpr int kLinearFixed = 7000;
+// The tile with the least estimated time: rounds of workgroups on the XCD that
+// gets the most of them (one to a CU, 32 CUs; column tiles go round the XCDs
+// whole), each a fixed part and its stages.  Nanoseconds of both by least
+// squares over 550 to 940 one-round launches a tile (64 tiles and more; 1 to 512
+// rows, 512 to 16384 weight rows, 8 to 32 stages; rms residual 1.1 to 2.3 us).
+// The fixed part holds the launch, the first stages' way into LDS and the
+// stores; a stage is 25 to 27 bytes per clock into the CU.  On 1428 other random
+// sizes the pick is within 3 % of the fastest of the four tiles.  Rounds over
+// the whole chip's 256 CUs instead take 7 x 34 tiles (448 rows, 2160 columns)
+// for one round, though two XCDs get 35 of them: 13.3 us against 10.3.
+struct LinearTile { int bm, bn, fixed, stage; };
+constexpr LinearTile kLinearTiles[] = {
+    {64, 64, 2900, 260}, {128, 64, 3300, 350}, {128, 128, 4200, 520}, {128, 192, 5300, 680}};
 
 int pick_linear_tile(int M, int rows_w, int K) {
   int best = 0;
   int64_t cost = INT64_MAX;
   for (int i = 0; i < 4; ++i) {
     const LinearTile& t = kLinearTiles[i];
-    const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((rows_w + t.bn - 1) / t.bn);
-    const int64_t c = (tiles + 255) / 256 * (kLinearFixed + (int64_t)(K / LN_BK) * t.clk);
+    const int64_t per_xcd = (int64_t)((M + t.bm - 1) / t.bm) * (((rows_w + t.bn - 1) / t.bn + 7) / 8);
+    const int64_t c = (per_xcd + 31) / 32 * (t.fixed + (int64_t)(K / LN_BK) * t.stage);
     if (c < cost) {
       cost = c;
       best = i;
@@ -280,6 +285,12 @@ void launch_linear_tile(const LinearArgs& a, hipStream_t stream) {
 }  // namespace gr
 
 using namespace gr;
+
+extern "C" int gr_linear_tile(int num_tokens, int out_features, int in_features, int swiglu) {
+  if (num_tokens < 1 || out_features < 1 || out_features > (1 << 28) || in_features < 1) return 0;
+  const LinearTile& t = kLinearTiles[pick_linear_tile(num_tokens, (swiglu ? 2 : 1) * out_features, in_features)];
+  return t.bm * 1000 + t.bn;
+}
 
 extern "C" gr_status_t gr_linear(void* out, int64_t out_stride, const void* x, int64_t x_stride, const void* w,
                                  int64_t w_stride, int num_tokens, int out_features, int in_features, int swiglu,

@@ -98,6 +98,7 @@ SIGNATURES = {
         _I, _I, _I, _F, _I, _P, _P,     # Hq, Hkv, head_dim, eps, dtype, dev_status, stream
     ]),
     "gr_linear": (_I, [_P, _L, _P, _L, _P, _L, _I, _I, _I, _I, _I, _I, _P]),
+    "gr_linear_tile": (_I, [_I, _I, _I, _I]),
     "gr_silu_mul": (_I, [_P, _L, _P, _L, _I, _I, _I, _P]),
     "gr_reshape_and_cache": (_I, [
         _P, _L, _P, _L, _P, _P, _L, _L, _L, _L, _P, _I, _I, _I, _I, _I, _P, _P,
