@@ -1,6 +1,8 @@
-"""gr_linear's choice of tile, without a GPU."""
+"""gr_linear's choice of tile and the decoder's choice of gr_linear, without a GPU."""
 
 import pytest
+
+from vllm_gr_amd.v1.sid_decoder import _own_sizes
 
 
 def _tile(lib, m, n, k, swiglu=0):
@@ -24,3 +26,17 @@ def test_tiles_fill_each_xcd_in_one_round(built_lib, m, n, k, swiglu):
 def test_tile_arguments(built_lib):
     assert built_lib.gr_linear_tile(0, 64, 512, 0) == built_lib.gr_linear_tile(4, 0, 512, 0) == 0
     assert _tile(built_lib, 1, 16, 512) == (64, 64)
+
+
+@pytest.mark.parametrize("m,rows,k,swiglu", [(384, 4096, 2048, False), (368, 3072, 2048, False), (272, 6144, 2048, False),
+                                             (512, 65536, 1024, False), (136, 32768, 2048, False), (64, 1024, 2048, False),
+                                             (448, 2 * 14336, 2048, True), (640, 4096, 2048, False), (8, 2048, 6144, False)])
+def test_sizes_where_the_library_measured_faster_stay_there(m, rows, k, swiglu):
+    assert not _own_sizes(m, rows, k, swiglu)
+
+
+@pytest.mark.parametrize("m", [1, 8, 100, 200, 512])
+def test_decode_step_projections_are_own(m):
+    """qkv, gate_up and lm_head of the 2048-feature decoder (o: but for 64 and 128 rows)."""
+    for rows, swiglu in ((4096, False), (2048, False), (12288, True), (8192, False)):
+        assert _own_sizes(m, rows, 2048, swiglu)

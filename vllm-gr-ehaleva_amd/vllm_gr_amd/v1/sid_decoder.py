@@ -14,9 +14,9 @@ from N(0, std) -- there are no checkpoints here:
   residual add;
 * final RMSNorm; logits = lm_head products in ``cfg.dtype``, widened to float32.
 
-The projections of up to 512 rows from at most 2048 features -- a decode
-step's qkv, o, gate_up (with its SiLU gate) and lm_head -- are gr_linear; the
-others are ``torch.nn.functional.linear`` (hipBLASLt on ROCm).  The
+The projections of a decode step's qkv, o, gate_up (with its SiLU gate) and
+lm_head are gr_linear where that is the faster (up to 512 rows, from at most 2048
+features: ``_own_sizes``); the others are ``torch.nn.functional.linear`` (hipBLASLt on ROCm).  The
 elementwise stages are fused HIP kernels (include/gr_decoder.h): residual add
 + RMSNorm, per-head q/k RMSNorm + rotary + K/V cache write through the slot
 mapping, and the SiLU-gated product.  Attention is
@@ -133,12 +133,46 @@ def _plain(*ts: torch.Tensor) -> bool:
             and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
 
 
+def _own_sizes(m: int, rows: int, k: int, swiglu: bool) -> bool:
+    """Whether gr_linear takes a projection of ``m`` rows by ``rows`` weight rows
+    of ``k`` features.
+
+    Measured with cold weights over 1 to 512 rows, 512 to 151936 weight rows and
+    512 to 2048 features, own time / the library's (SwiGLU: its product and the
+    gate kernel's):
+
+    * workgroups that fill the chip once (128 x 192 tiles, column tiles whole on
+      one of the 8 XCDs of 32 CUs) and SwiGLU, 0.37 to 0.91, or at most 1024
+      features, 0.44 to 1.00 (of random sizes 1 in 100 up to 1.17).  In more rounds
+      0.75 to 1.60, SwiGLU 0.43 to 1.35;
+    * one round and more features: 0.51 to 1.00, but not where few columns leave
+      most CUs idle and the rows fill the library's tiles (33 to 128 rows: 512
+      columns 0.97 to 1.04, 1024 0.85 to 1.09, 2048 at 64 and 128 rows 0.99 to
+      1.03), and not around its best fits past 1536 features (337 to 384 rows, 3072
+      and 4096 columns 1.01 to 1.08; 257 to 315 rows, 5664 to 6512 columns 1.04 to
+      1.10, though 0.80 to 0.89 at 320 to 340);
+    * up to 100 rows the weights' way from memory is the time, also in more
+      rounds: 0.55 to 0.98 past 1024 features;
+    * above the limits: 768 rows, SwiGLU 2048 in, 6144 out 53 us against 44; 6144
+      in, 2048 out, 8 rows 21 against 12."""
+    if m > 512 or k > 2048:
+        return False
+    one_round = -(-m // 128) * -(-rows // (8 * 192)) <= 32
+    if swiglu or k <= 1024:
+        return one_round
+    if not one_round:
+        return m <= 100
+    if m <= 32:
+        return True
+    if m <= 128:
+        return rows > 2048 or (rows > 1024 and m % 64 != 0)
+    if k > 1536 and 256 < m <= 384 and 2560 < rows < 8192:
+        return rows <= 5120 and m <= 336
+    return rows > 512
+
+
 def _own_linear(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> bool:
-    """Whether gr_linear takes a projection.  Its gains are at decode-step row
-    counts and shallow depths: at 768 rows SwiGLU (2048 in, 6144 out) takes 55
-    us against the library's 51, at 512 32 against 37; 6144 in, 2048 out, 8 rows
-    21 against 12."""
-    return x.shape[0] <= 512 and w.shape[1] <= 2048 and ops.linear_supported(x, w, swiglu)
+    return _own_sizes(x.shape[0], *w.shape, swiglu) and ops.linear_supported(x, w, swiglu)
 
 
 def _linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
