@@ -264,6 +264,9 @@ __global__ __launch_bounds__(R5_THREADS) void decode_row512(DecodeArgs a, int un
       t_beam[wave][buf][lane] = ok ? k.beam : -2;
       t_pos[wave][buf][lane] = k.pos;
     }
+    // other lanes of the wave read these entries: nothing moves across
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   };
   uint8_t* ktile = tiles + wave * REGION;
   // tile rows 2 i, 2 i + 1 by load i: position p of row key holds chunk p ^ (key % 16)
