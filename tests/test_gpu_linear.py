@@ -10,7 +10,7 @@ fp16), and SwiGLU's exponential and quotient a few float32 units."""
 import pytest
 import torch
 
-from vllm_gr_amd import ops
+from vllm_gr_amd import _C, ops
 from vllm_gr_amd.v1.sid_decoder import DecoderConfig, SidDecoder, init_weights
 
 pytestmark = pytest.mark.gpu
@@ -39,6 +39,20 @@ def test_linear(device, dtype, M, N, K):
     dg, du = own[:, :N] + half * gate.abs(), own[:, N:] + half * up.abs()
     tol = sw.abs() * (1.01 * half + 2.0 ** -21) + 1.01 * (1.1 * dg * up.abs() + gate.abs() * du) + 2.0 ** -24
     assert ((z.double() - sw).abs() <= tol).all()
+
+
+# (rows, columns, SwiGLU, its tile): every tile of either form, with rows and columns left over
+TILES = [(65, 80, 0, (64, 64)), (300, 4112, 0, (128, 64)), (301, 8144, 0, (128, 128)), (500, 8208, 0, (128, 192)),
+         (65, 80, 1, (64, 64)), (301, 2064, 1, (128, 64)), (300, 4112, 1, (128, 128)), (500, 6128, 1, (128, 192))]
+
+
+@pytest.mark.parametrize("K", [576, 640])  # an odd and an even number of stages past every pipeline's first
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,swiglu,tile", TILES)
+def test_linear_every_tile(device, dtype, M, N, swiglu, tile, K):
+    assert _C.lib().gr_linear_tile(M, N, K, swiglu) == 1000 * tile[0] + tile[1]
+    assert M % tile[0] and (N * (1 + swiglu)) % tile[1]
+    test_linear(device, dtype, M, N, K)
 
 
 def test_linear_refuses(device):
