@@ -145,3 +145,74 @@ def test_row512_small_weight_of_a_large_value(device, dtype, D):
     sub = 2.0 ** -25 if dtype == torch.float16 else 0.0
     own = D * 2.0 ** -24 * s.numpy() / 2 + 2.0 ** -20
     assert (np.abs(out - ref) <= (1.01 * HALF_ULP[dtype] + own) * np.abs(ref) + sub).all(), (np.abs(out - ref) / ref).max()
+
+
+def _padded(t, pad, dims):
+    """t's values in a tensor whose given dims are `pad` longer, viewed at t's shape."""
+    shape = [n + (pad if i in dims else 0) for i, n in enumerate(t.shape)]
+    return torch.zeros(shape, dtype=t.dtype, device=t.device)[tuple(slice(n) for n in t.shape)].copy_(t)
+
+
+@pytest.mark.parametrize("dtype,D", DTYPES)
+def test_row512_layouts(device, dtype, D):
+    """Caches padded per head or held head-major, strided q and out, suffixes
+    that start inside their blocks: the same bits as the packed form, which is
+    checked against the oracle.  Bases or strides off the 16-byte grid: the
+    generic kernel's bits."""
+    wl = workloads.make_decode(R=2, W=5, P=75, L=(3, 17), Hq=8, Hkv=2, D=D, dtype=dtype, input_scale=1.0, seed=11,
+                               suffix_blocks=3)
+    start = torch.randint(0, 16, (10,), dtype=torch.int32, generator=torch.Generator().manual_seed(1))
+    kv = wl.kv_cache.double().numpy()
+    ref, _ = oa.beam_attention_cascade(
+        wl.q.double().numpy(), kv[0], kv[1], wl.prefix_bt.numpy(), wl.prefix_len.numpy(), wl.beam_start.numpy(),
+        wl.suffix_bt.numpy(), wl.suffix_len.numpy(), start.numpy(), q_per_beam=1, scale=wl.scale, block_size=16)
+    d, ch = wl.to(device), 16 // wl.q.element_size()
+    start = start.to(device)
+
+    def run(q, kvc, out, kernel="auto"):
+        ops.set_decode_kernel(kernel)
+        try:
+            ops.beam_attn_decode(q, kvc[0], kvc[1], d.prefix_bt, d.prefix_len, d.beam_start, d.suffix_bt, d.suffix_len,
+                                 start, scale=d.scale, max_beams_per_req=5, out=out)
+            torch.cuda.synchronize()
+        finally:
+            ops.set_decode_kernel("auto")
+        return out.contiguous()
+
+    new = lambda: torch.empty_like(d.q)
+    base = run(d.q, d.kv_cache, new())
+    assert (np.abs(base.double().cpu().numpy() - ref) <= _bound(ref, wl, dtype)).all()
+    wide = lambda t, pad: _padded(t.flatten(1), pad, (1,)).unflatten(1, t.shape[1:])  # token stride Hq D + pad
+    for name, q, kvc, out in (
+            ("padded heads", d.q, _padded(d.kv_cache, ch, (4,)), new()),
+            ("padded tokens", d.q, _padded(d.kv_cache, 1, (2, 3)), new()),
+            ("head-major", d.q, d.kv_cache.transpose(2, 3).contiguous().transpose(2, 3), new()),
+            ("strided q, out", wide(d.q, ch), d.kv_cache, wide(new(), 3 * ch))):
+        assert torch.equal(run(q, kvc, out), base), name
+    gen = run(d.q, d.kv_cache, new(), "generic")
+    off = torch.zeros(d.kv_cache.numel() + 1, dtype=dtype, device=device)[1:].view_as(d.kv_cache).copy_(d.kv_cache)
+    for name, q, kvc, out in (
+            ("unaligned heads", d.q, _padded(d.kv_cache, 1, (4,)), new()),
+            ("unaligned base", d.q, off, new()),
+            ("unaligned q", wide(d.q, 1), d.kv_cache, new()),
+            ("unaligned out", d.q, d.kv_cache, wide(new(), 1))):
+        assert torch.equal(run(q, kvc, out), gen), name
+
+
+@pytest.mark.parametrize("dtype,D", DTYPES)
+def test_row512_weights_of_every_size(device, dtype, D):
+    """Scores spread over some 30: tiles with large weights only and tiles with
+    weights far below 2^-12 of the row's largest, in one row.
+
+    Bound: as above, plus the scores' float32 sums of D products (errors of both
+    signs: 4 sqrt(D) 2^-24 of the largest score, 20) on the largest |v|."""
+    wl = workloads.make_decode(R=2, W=11, P=500, L=(1, 6), Hq=8, Hkv=2, D=D, dtype=dtype, input_scale=2.0, seed=17)
+    wl.kv_cache[0, wl.prefix_bt[:, ::2].long().flatten()] /= 8  # every other block: near ties
+    out, lse = _run(wl, device)
+    kv = wl.kv_cache.double().numpy()
+    ref, ref_lse = oa.beam_attention_cascade(
+        wl.q.double().numpy(), kv[0], kv[1], wl.prefix_bt.numpy(), wl.prefix_len.numpy(), wl.beam_start.numpy(),
+        wl.suffix_bt.numpy(), wl.suffix_len.numpy(), q_per_beam=1, scale=wl.scale, block_size=16)
+    own = 4 * D ** 0.5 * 2.0 ** -24 * 20 * float(wl.kv_cache[1].abs().max())
+    assert (np.abs(out - ref) <= _bound(ref, wl, dtype) + own).all(), np.abs(out - ref).max()
+    assert np.abs(lse - ref_lse).max() <= 1e-4
