@@ -136,14 +136,78 @@ def test_attention_kernels_keep_no_stack():
 
 
 def test_path_kernels_outside_attention_keep_no_stack():
-    """The pruning, fork and split-merge kernels of the decode step hold
-    their state in registers and LDS: none of them touches scratch (the
+    """The pruning, fork and split-merge kernels of the decode step, the decode
+    of 512-byte rows and the projections hold their state in registers and LDS: none of them touches scratch (the
     very wide requests' one-pass merge, which keeps 16 candidates per thread,
     is the exception and is not checked)."""
     sizes = _scratch_sizes()
-    names = ("prune_rows", "prune_merge_part", "prune_merge_lists", "beam_fork", "beam_append",
-             "split_merge", "catalog_advance")
+    names = ("prune_rows", "prune_slice_max", "prune_slice_sum", "prune_merge_part", "prune_merge_lists", "beam_fork",
+             "beam_append", "split_merge", "catalog_advance", "decode_row512", "linear_k")
     found = {k: v for k, v in sizes.items() if any(n in k for n in names)}
     for n in names:
         assert any(n in k for k in found), n
     assert all(v == 0 for v in found.values()), {k: v for k, v in found.items() if v}
+
+
+VMEM = re.compile(r"^(global|buffer|flat|scratch)_(load|store|atomic)")
+
+
+def _kernels(text, name):
+    """Kernel -> its instructions (mnemonic and operands), for kernels whose name holds `name`."""
+    out = {}
+    for part in re.split(r"\n(?=[0-9a-f]+ <)", text):
+        m = re.match(r"[0-9a-f]+ <(.*)>:", part)
+        if m and name in m.group(1):
+            out[m.group(1)] = [l.split("//")[0].strip() for l in part.split("\n")[1:] if l.strip()]
+    return out
+
+
+def _row512_loads_before_wait(code):
+    """For each wait that leaves 16 vector-memory operations in flight: the
+    16-byte loads into registers issued before it in its straight line."""
+    counts = []
+    for i, ins in enumerate(code):
+        if ins != "s_waitcnt vmcnt(16)":
+            continue
+        n = 0
+        for prev in reversed(code[:i]):
+            if prev.startswith(("s_cbranch", "s_branch")) or "_load_lds_" in prev:
+                break
+            n += prev.startswith("global_load_dwordx4 ")
+        counts.append(n)
+    return counts
+
+
+def _linear_counted(code):
+    """Vector-memory operations up to the last barrier other than transfers into LDS."""
+    last = max(i for i, ins in enumerate(code) if ins.startswith("s_barrier"))
+    return [ins for ins in code[:last] if VMEM.match(ins) and not ins.startswith("global_load_lds_dwordx4 ")]
+
+
+def test_hand_counted_waits_count_what_they_assume():
+    """Transfers into LDS are waited for by counts.  decode_row512 waits until 16
+    operations are in flight, the V loads issued after the K tile's transfers:
+    with fewer of them after the last transfer, part of the tile would not be in
+    LDS yet.  linear_k counts whole stages of transfers: no other vector-memory
+    operation may be among them."""
+    text = _disassembly()
+    rows = _kernels(text, "decode_row512")
+    assert len(rows) == 6
+    for k, code in rows.items():
+        counts = _row512_loads_before_wait(code)
+        assert counts and all(n >= 16 for n in counts), (k, counts)
+    lin = _kernels(text, "linear_k")
+    assert len(lin) == 16
+    for k, code in lin.items():
+        assert not _linear_counted(code), (k, _linear_counted(code)[:3])
+
+
+def test_wait_checks_flag_a_miscount():
+    """The checks themselves: a V load moved below the wait, and a load among the counted transfers."""
+    loads = ["global_load_dwordx4 v[0:3], v[8:9], off"] * 16
+    wait, lds = "s_waitcnt vmcnt(16)", "global_load_lds_dwordx4 v[0:1], off"
+    assert _row512_loads_before_wait([lds] + loads + [wait]) == [16]
+    assert _row512_loads_before_wait([lds] + loads[1:] + [wait, loads[0]]) == [15]
+    assert _row512_loads_before_wait(loads[:4] + [lds] + loads[4:] + [wait]) == [12]
+    assert _linear_counted([lds, "s_barrier", "global_store_dwordx2 v0, v[0:1], s[0:1]"]) == []
+    assert len(_linear_counted([lds, "global_load_dword v0, v1, s[0:1]", "s_barrier"])) == 1
