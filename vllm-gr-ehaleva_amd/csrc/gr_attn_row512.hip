@@ -2,8 +2,10 @@
 // head_dim 128, bf16 / fp16 at head_dim 256), in float32 precision throughout.
 //
 // What bounds it: these shapes are small (tens of megabytes of KV at most a
-// request), so the time is the chain of one workgroup: its share of the keys
-// through the CU's 64 bytes per clock, or, in float32, the float32 MFMA rate.
+// request), so the time is the chain of one workgroup: per tile of a wave the
+// loads of V, then of the next K (each CU takes its 1.1 MB at 45 GB/s in the
+// head_dim 256 case below; streams reach 95 and more), or, in float32, the
+// float32 MFMA rate.
 // The split is therefore over rows and, inside the workgroup, over keys: a
 // workgroup owns 16 query rows of one (request, KV head) -- the smallest MFMA
 // tile, for the most workgroups -- and its 8 waves take every eighth tile of 32
@@ -24,7 +26,8 @@
 //    float32 values are operands as loaded; 16-bit ones need an 8 x 8 transpose
 //    inside the lane (32 byte permutes per chunk).
 // K tiles go straight from global memory into the wave's own LDS tile (chunks
-// XOR-swizzled by the key, so the A reads touch every bank once); the next
+// XOR-swizzled by the key, so the A reads touch every bank once; the 16-bit
+// merge's writes at the end take 4 cycles more each than they need); the next
 // tile's transfer runs under this tile's softmax and PV, and V arrives in
 // registers under QK.  No barrier inside the loop: a wave reads only its own
 // tiles.

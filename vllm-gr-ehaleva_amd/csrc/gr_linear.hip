@@ -26,7 +26,8 @@
 //   out 2048      8.2 ->  7.9   8.9 ->  8.5   9.6 ->  8.7  11.0 ->  9.1  11.4 ->  9.8
 //   SwiGLU 6144  18.7 -> 13.2  20.4 -> 15.7  31.1 -> 22.9  37.8 -> 29.4  39.2 -> 32.8
 //   out 8192     14.1 -> 11.5  14.8 -> 14.2  18.2 -> 16.0  24.4 -> 22.8  27.8 -> 24.1
-// (SwiGLU against the library's product and the separate gate kernel.)
+// (SwiGLU against the library's product and the separate gate kernel.  The
+// decoder leaves sizes like 384 rows x 4096 columns to the library.)
 // All row tiles of a column tile run on one XCD: the weights, which come from
 // HBM, are then read into one L2 only.
 #include "gr_decoder.h"
